@@ -63,6 +63,64 @@ def test_quant_bitwise(hip_lib):
     assert fn(None, None, None, 4, 64, 16, None) == ve.VK_ERROR_UNSUPPORTED
 
 
+@pytest.mark.parametrize("hidden", [32, 64, 96, 544, 2048, 4096 + 32])
+def test_quant_widths_and_magnitudes_bitwise(hip_lib, hidden):
+    """Rows that share a wavefront, end inside a batch of loads or take several, at magnitudes
+    around the ends of the packed routine's range of scale bytes (4 .. 143) and beyond, with
+    every value near a rounding threshold."""
+    fn = hip_lib.vk_hip_mxfp4_moe_quant
+    fn.restype = _I
+    fn.argtypes = [_P, _P, _P, _I, _I, _I, _P]
+    M = 97
+    rng = np.random.default_rng(hidden)
+    near = np.array([.125, .625, 1.25, 1.75, 2.5, 3.0], np.float32)
+    steps = rng.integers(-2, 3, (M, hidden))
+    bits = synth.f32_to_bf16_bits(near[rng.integers(0, 6, (M, hidden))]).astype(np.int64) + steps
+    exps = np.r_[np.arange(1 - 127, 8 - 127), np.arange(139 - 127, 148 - 127), rng.integers(-100, 100, M)][:M]
+    vals = synth.bf16_bits_to_f32(bits.astype(np.uint16)).astype(np.float64) * 2.0 ** exps[:, None]
+    vals *= rng.choice([-1.0, 1.0], (M, hidden))
+    A = synth.f32_to_bf16_bits(vals.astype(np.float32))
+    A[rng.random((M, hidden)) < 0.02] = 0x8001           # a negative subnormal among them
+    A[11, hidden - 1] = 0x7FC0                           # a NaN, an infinity, a group of zeros
+    A[12, 0] = 0xFF80
+    A[13, :32] = 0x8000
+    packed = torch.zeros((M, hidden // 2), dtype=torch.uint8, device=dev())
+    scales = torch.zeros((M, hidden // 32), dtype=torch.uint8, device=dev())
+    d_A = to_dev(A)
+    assert fn(d_A.data_ptr(), packed.data_ptr(), scales.data_ptr(), M, hidden, 32, None) == 0
+    torch.cuda.synchronize()
+    rp, rs = oracle.mxfp4_moe_quant(A)
+    assert np.array_equal(scales.cpu().numpy(), rs) and np.array_equal(packed.cpu().numpy(), rp)
+
+
+@pytest.mark.parametrize("top_k", [1, 2, 3, 4, 6, 8])
+def test_scatter_reduce_on_a_used_workspace(hip_lib, top_k):
+    """The table of sorted positions holds what an earlier call left there: flat indices without
+    a sorted row (a quarter of the experts is another rank's) add nothing, whatever their
+    entries say."""
+    sr = hip_lib.vk_hip_mxfp4_moe_scatter_reduce
+    sr.restype = _I
+    sr.argtypes = [_P, _P, _P, _P, _I, _I, _I, _I, _P, ctypes.c_size_t, _P]
+    rng = np.random.default_rng(top_k)
+    M, E, width = 53, 16, 132
+    ids = np.stack([rng.permutation(E)[:top_k] for _ in range(M)]).astype(np.int32)
+    emap = np.where(np.arange(E) % 4 == 1, -1, np.cumsum(np.arange(E) % 4 != 1) - 1).astype(np.int32)
+    sids, _, em = oracle.moe_align_block_size_with_map(ids.ravel(), E, 16, emap)
+    sids = sids[:em].copy()
+    partial = rng.standard_normal((em, width)).astype(np.float32)
+    tws = rng.random(em).astype(np.float32)
+    base = rng.standard_normal((M, width)).astype(np.float32)
+    ref = oracle.mxfp4_moe_scatter_reduce(partial, tws, sids, M, top_k, out=base.copy())
+    d_p, d_w, d_s = to_dev(partial), to_dev(tws), to_dev(sids)
+    for garbage in (np.full(M * top_k, -1), np.arange(M * top_k) % em, np.full(M * top_k, em),
+                    rng.integers(-2 ** 31, 2 ** 31, M * top_k)):
+        ws, out = to_dev(garbage.astype(np.int32)), to_dev(base.copy())
+        assert sr(d_p.data_ptr(), d_w.data_ptr(), d_s.data_ptr(), out.data_ptr(), M, width, top_k, em,
+                  ws.data_ptr(), ws.numel() * 4, None) == 0
+        torch.cuda.synchronize()
+        assert np.array_equal(out.cpu().numpy().view(np.uint32), ref.view(np.uint32))
+
+
 def test_sorted_quant_and_scatter_reduce_bitwise(hip_lib):
     sq = hip_lib.vk_hip_mxfp4_moe_sorted_quant
     sq.restype = _I

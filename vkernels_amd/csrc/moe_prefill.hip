@@ -283,62 +283,196 @@ __global__ __launch_bounds__(256) void split_rows_fp6_kernel(const uint16_t* __r
 //   only for m = 1.5), at least 1;
 //   code = nearest of {0, .25, 1, 1.5, 2, 3} to |a| / 2^(s-127), ties to the larger
 //   (thresholds .125, .625, 1.25, 1.75, 2.5), sign bit set when a / scale < 0.
-// d: the 32 values, two per dword; codes: 4 dwords, low nibble = even k.
+//
+// The four lanes of a quad hold a group, 8 values each, so that loads and stores are
+// contiguous over the lanes.  The kernels are bound by vector arithmetic before they are
+// bound by memory (2 bytes in and half a byte out per value), so the codes come from
+// packed 16-bit integer operations on the bit patterns, which order like the magnitudes:
+// with z = (bits - bits(.125 x 2^(s-127)) + 32) / 32, clamped at zero, the thresholds
+// are z = 1, 10, 14, 16, 18, and the code is [z >= 1] + [z >= 10] + floor(max(z - 12, 0) / 2),
+// 8 instructions a value instead of the 20 of a chain of float comparisons.  Groups with a
+// NaN, or a scale so small or large that a threshold or a product leaves the normal
+// numbers (s outside 4 .. 143), take that chain.  4096 wide, 32768 sorted rows of which
+// 24576 routed: 72 -> 42 us.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ void quant_group32(const uint32_t (&d)[16], uint32_t& sb, uint32_t (&codes)[4]) {
-  // (bit patterns of non-negative floats order like the floats; a NaN counts as zero)
-  uint32_t bits = 0u;
+typedef __attribute__((ext_vector_type(2))) uint16_t u16x2;
+
+__device__ __forceinline__ uint32_t pk_sub_sat(uint32_t a, uint32_t b) {
+  union { uint32_t u; u16x2 h; } x, y;
+  x.u = a;
+  y.u = b;
+  x.h = __builtin_elementwise_sub_sat(x.h, y.h);
+  return x.u;
+}
+__device__ __forceinline__ uint32_t pk_min(uint32_t a, uint32_t b) {
+  union { uint32_t u; u16x2 h; } x, y;
+  x.u = a;
+  y.u = b;
+  x.h = __builtin_elementwise_min(x.h, y.h);
+  return x.u;
+}
+__device__ __forceinline__ uint32_t pk_max(uint32_t a, uint32_t b) {
+  union { uint32_t u; u16x2 h; } x, y;
+  x.u = a;
+  y.u = b;
+  x.h = __builtin_elementwise_max(x.h, y.h);
+  return x.u;
+}
+__device__ __forceinline__ uint32_t pk_shr(uint32_t a, int n) {
+  union { uint32_t u; u16x2 h; } x;
+  x.u = a;
+  x.h = x.h >> (uint16_t)n;
+  return x.u;
+}
+
+__device__ __forceinline__ uint32_t quad_max(uint32_t m) {
+  m = max(m, (uint32_t)__builtin_amdgcn_mov_dpp((int)m, 0xB1, 0xF, 0xF, true));
+  return max(m, (uint32_t)__builtin_amdgcn_mov_dpp((int)m, 0x4E, 0xF, 0xF, true));
+}
+
+// The scale byte of a group whose largest magnitude has these bits (finite, not zero).
+__device__ __forceinline__ uint32_t quant_scale_byte(uint32_t bits) {
+  const uint32_t ex = bits >> 7;
+  const int s = (int)ex - ((bits & 0x7Fu) <= 0x40u ? 1 : 0);
+  return (uint32_t)(ex == 0u || s < 1 ? 1 : s);
+}
+
+// The 8 codes of two-per-dword values v under scale byte s in 4 .. 143, no NaN among them.
+__device__ __forceinline__ uint32_t quant8_packed(const u32x4& v, uint32_t s) {
+  uint32_t ones = 0x00010001u;
+  __asm__("" : "+s"(ones));  // (a minimum with a known 1 becomes two comparisons and selections)
+  const uint32_t base = ((s - 3u) << 7) - 32u;  // 32 below the bits of .125 x 2^(s-127)
+  const uint32_t base2 = base | (base << 16);
+  uint32_t b[4];
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    uint32_t lo = d[i] & 0x7FFFu, hi = (d[i] >> 16) & 0x7FFFu;
+  for (int j = 0; j < 4; ++j) {
+    const uint32_t mag = v[j] & 0x7FFF7FFFu;
+    const uint32_t z = pk_shr(pk_sub_sat(mag, base2), 5);
+    const uint32_t c = pk_min(z, ones) + pk_min(pk_sub_sat(z, 0x00090009u), ones) +
+                       pk_shr(pk_sub_sat(z, 0x000C000Cu), 1);
+    const uint32_t neg = pk_shr(v[j], 15) & pk_min(mag, ones);  // (-0 has no sign bit)
+    const uint32_t n = c | (neg << 3);
+    b[j] = n | (n >> 12);  // the two codes in the low byte
+  }
+  const uint32_t lo = __builtin_amdgcn_perm(b[1], b[0], 0x0C0C0400u);
+  const uint32_t hi = __builtin_amdgcn_perm(b[3], b[2], 0x0C0C0400u);
+  return lo | (hi << 16);
+}
+
+// The same for any finite group and any scale byte; a NaN gets code 5.
+__device__ __forceinline__ uint32_t quant8_any(const u32x4& v, uint32_t s) {
+  // a / 2^(s-127) as a product with 2^(127-s), exact (the rounding at underflow included)
+  const float inv = s <= 253u ? __uint_as_float((254u - s) << 23) : __uint_as_float(0x00400000u);
+  uint32_t word = 0u;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const uint32_t dw = v[i >> 1];
+    const float x = __fmul_rn(__uint_as_float((i & 1) ? (dw & 0xFFFF0000u) : (dw << 16)), inv);
+    const float m = fabsf(x);
+    uint32_t mag = 5u;              // also what a NaN gets: every comparison is false
+    if (m < 0.125f) mag = 0u;
+    else if (m < 0.625f) mag = 1u;
+    else if (m < 1.25f) mag = 2u;
+    else if (m < 1.75f) mag = 3u;
+    else if (m < 2.5f) mag = 4u;
+    if (x < 0.0f) mag |= 8u;
+    word |= mag << (4 * i);
+  }
+  return word;
+}
+
+// Codes of this lane's 8 values and the scale byte of the quad's 32 (every lane of a quad
+// calls this together).  False: sb and codes are not the group's, quant_quad_any takes it.
+__device__ __forceinline__ bool quant_quad(const u32x4& v, uint32_t& sb, uint32_t& codes) {
+  uint32_t m = pk_max(pk_max(v[0] & 0x7FFF7FFFu, v[1] & 0x7FFF7FFFu), pk_max(v[2] & 0x7FFF7FFFu, v[3] & 0x7FFF7FFFu));
+  m = quad_max(max(m & 0xFFFFu, m >> 16));
+  sb = quant_scale_byte(m);
+  // (m beyond the infinity's bits: a NaN is in the group.  m zero or an infinity: below 4 or
+  // beyond 143 as well)
+  const bool packed = m <= 0x7F80u && sb - 4u <= 139u;
+  codes = quant8_packed(v, sb);
+  return packed;
+}
+
+__device__ __forceinline__ void quant_quad_any(const u32x4& v, uint32_t& sb, uint32_t& codes) {
+  uint32_t bits = 0u;  // a NaN counts as zero
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    uint32_t lo = v[i] & 0x7FFFu, hi = (v[i] >> 16) & 0x7FFFu;
     if (lo > 0x7F80u) lo = 0u;
     if (hi > 0x7F80u) hi = 0u;
     bits = max(bits, max(lo, hi));
   }
-  const uint32_t ex = bits >> 7, mant = bits & 0x7Fu;
-  if (ex == 0xFFu || bits == 0u) {
+  bits = quad_max(bits);
+  if (bits == 0u || bits == 0x7F80u) {
     sb = 0xFFu;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) codes[j] = 0u;
-    return;
+    codes = 0u;
+  } else {
+    sb = quant_scale_byte(bits);
+    codes = quant8_any(v, sb);
   }
-  int s = (int)ex - (mant <= 0x40u ? 1 : 0);
-  if (ex == 0u || s < 1) s = 1;
-  sb = (uint32_t)s;
-  // a / 2^(s-127) as a product with 2^(127-s), exact (the rounding at underflow included)
-  const float inv = s <= 253 ? __uint_as_float((uint32_t)(254 - s) << 23) : __uint_as_float(0x00400000u);
+}
+
+// Quantises the 8-value pieces first, first + step, ... of a row (pieces, step: whole quads;
+// every lane of the row's `step` lanes calls this): load(i) -> the piece's values,
+// store(i, codes, scale byte).  A few loads are issued together (one at a time is a round
+// trip to memory for every 8 values); the groups the packed routine does not take are done
+// over afterwards, where they occur, so that their code stands here once and out of the way.
+template <typename Load, typename Store>
+__device__ __forceinline__ void quant_row(int first, int step, int pieces, Load load, Store store) {
+  constexpr int kBatch = 4;
+  for (int i0 = first; i0 < pieces; i0 += kBatch * step) {
+    u32x4 v[kBatch];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    uint32_t word = 0u;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const uint32_t dw = d[j * 4 + (i >> 1)];
-      const float a = __uint_as_float((i & 1) ? (dw & 0xFFFF0000u) : (dw << 16));
-      const float x = __fmul_rn(a, inv);
-      const float v = fabsf(x);
-      uint32_t mag = 5u;              // also what a NaN gets: every comparison is false
-      if (v < 0.125f) mag = 0u;
-      else if (v < 0.625f) mag = 1u;
-      else if (v < 1.25f) mag = 2u;
-      else if (v < 1.75f) mag = 3u;
-      else if (v < 2.5f) mag = 4u;
-      if (x < 0.0f) mag |= 8u;
-      word |= mag << (4 * i);
+    for (int j = 0; j < kBatch; ++j) {
+      v[j] = u32x4{0u, 0u, 0u, 0u};
+      if (i0 + j * step < pieces) v[j] = load(i0 + j * step);
     }
-    codes[j] = word;
+    bool all = true;
+#pragma unroll
+    for (int j = 0; j < kBatch; ++j) {
+      if (i0 + j * step >= pieces) break;
+      uint32_t sb, codes;
+      if (quant_quad(v[j], sb, codes)) store(i0 + j * step, codes, sb);
+      else all = false;
+    }
+    if (all) continue;
+#pragma unroll 1
+    for (int i = i0; i < min(i0 + kBatch * step, pieces); i += step) {
+      const u32x4 w = load(i);
+      uint32_t sb, codes;
+      quant_quad_any(w, sb, codes);  // (any group: the same codes where the packed routine has been)
+      store(i, codes, sb);
+    }
   }
+}
+
+// Lanes that share a row (a power of two, as many as the row has pieces of 8 values, at
+// most a wavefront): short rows do not leave the rest of the wavefront idle.
+__host__ __device__ constexpr int quant_lane_bits(int pieces) {
+  int bits = 2;
+  while (bits < 6 && (1 << bits) < pieces) ++bits;
+  return bits;
+}
+static inline dim3 quant_grid(int rows, int pieces) {
+  const int per_group = 4 * (64 >> quant_lane_bits(pieces));  // 4 wavefronts
+  return dim3((unsigned)((rows + per_group - 1) / per_group));
 }
 
 // Packed codes [rows, K/2] and scale bytes [rows, K/32] of bf16 rows: row r of the output
 // is x[r] (sorted_ids null) or x[sorted_ids[r] / top_k], a padding row (id outside
 // [0, n_flat)) giving zero codes and 0xFF scales (mxfp4_moe_sorted_quant,
-// moe_aux.cpp:171-209).  One lane per group of 32.
+// moe_aux.cpp:171-209).
 __global__ __launch_bounds__(256) void mxfp4_quant_kernel(const uint16_t* __restrict__ x,
                                                           const int32_t* __restrict__ sorted_ids,
                                                           uint8_t* __restrict__ packed,
-                                                          uint8_t* __restrict__ scales, int K,
+                                                          uint8_t* __restrict__ scales, int K, int rows,
                                                           int top_k, int n_flat) {
-  const size_t row = blockIdx.x;
+  const int pieces = K / 8;
+  const int bits = quant_lane_bits(pieces);
+  const int lane = threadIdx.x & 63;
+  const size_t row = (size_t)(blockIdx.x * 4 + (threadIdx.x >> 6)) * (size_t)(64 >> bits) + (size_t)(lane >> bits);
+  if (row >= (size_t)rows) return;
   const uint16_t* src = x + row * (size_t)K;
   bool pad = false;
   if (sorted_ids != nullptr) {
@@ -346,62 +480,70 @@ __global__ __launch_bounds__(256) void mxfp4_quant_kernel(const uint16_t* __rest
     pad = flat < 0 || flat >= n_flat;
     src = x + (size_t)(pad ? 0 : flat / top_k) * (size_t)K;
   }
-  for (int g = threadIdx.x; g < K / 32; g += 256) {
-    union { u32x4 q[4]; uint32_t d[16]; } in;
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      in.q[i] = pad ? u32x4{0u, 0u, 0u, 0u} : reinterpret_cast<const u32x4*>(src + (size_t)g * 32)[i];
-    uint32_t sb, codes[4];
-    quant_group32(in.d, sb, codes);
-    *reinterpret_cast<u32x4*>(packed + row * (size_t)(K / 2) + (size_t)g * 16) =
-        u32x4{codes[0], codes[1], codes[2], codes[3]};
-    scales[row * (size_t)(K / 32) + g] = (uint8_t)sb;
+  uint8_t* const prow = packed + row * (size_t)(K / 2);
+  uint8_t* const srow = scales + row * (size_t)(K / 32);
+  const int step = 1 << bits, first = lane & (step - 1);
+  auto store = [&](int i, uint32_t codes, uint32_t sb) {
+    *reinterpret_cast<uint32_t*>(prow + (size_t)i * 4) = codes;
+    if ((i & 3) == 0) srow[i >> 2] = (uint8_t)sb;
+  };
+  if (pad) {
+    for (int i = first; i < pieces; i += step) store(i, 0u, 0xFFu);
+    return;
   }
+  quant_row(first, step, pieces, [&](int i) { return *reinterpret_cast<const u32x4*>(src + (size_t)i * 8); }, store);
 }
 
 // The same quantisation as the split rows of the W4A4 mode: one plane of Kp bytes per
 // row, a block = the 32 codes moved onto the OCP code points (16 bytes), the scale byte
 // less one, 15 zero bytes; zero groups get a neutral scale.  row_bad[r] = 1 when a scale
-// byte is outside the range the scaled MFMA path takes.
+// byte is outside the range the scaled MFMA path takes.  8191 tokens x 6 rows of 1536:
+// 169 -> 59 us (4.1 TB/s) with as many rows a wavefront as it has lanes for (a workgroup per row left
+// four fifths of it idle) and the packed quantisation.
 __global__ __launch_bounds__(256) void quant_rows_w4_kernel(const uint16_t* __restrict__ x,
                                                             uint8_t* __restrict__ xq,
-                                                            uint8_t* __restrict__ row_bad, int K,
+                                                            uint8_t* __restrict__ row_bad, int K, int rows,
                                                             const int32_t* __restrict__ sorted_ids,
                                                             int n_flat, int32_t* __restrict__ fill,
                                                             int fill_n) {
   for (int i = (int)(blockIdx.x * 256 + threadIdx.x); i < fill_n; i += (int)(gridDim.x * 256)) fill[i] = -1;
   const int kp = mx_kp(K);
-  const size_t row = blockIdx.x;
-  if (sorted_ids != nullptr) {  // as split_rows_fp6_kernel: routed rows only (uniform per workgroup)
+  const int pieces = kp / 8;
+  const int bits = quant_lane_bits(pieces);
+  const int lane = threadIdx.x & 63;
+  const size_t row = (size_t)(blockIdx.x * 4 + (threadIdx.x >> 6)) * (size_t)(64 >> bits) + (size_t)(lane >> bits);
+  if (row >= (size_t)rows) return;
+  if (sorted_ids != nullptr) {  // as split_rows_fp6_kernel: routed rows only
     const int f = sorted_ids[row];
     if (f < 0 || f >= n_flat) return;
   }
   uint8_t* qrow = xq + row * (size_t)kp;
-  int bad = 0;
-  for (int b = threadIdx.x; b < kp / 32; b += 256) {
-    union { u32x4 q[4]; uint32_t d[16]; } in;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) in.q[i] = u32x4{0u, 0u, 0u, 0u};
-    if (b * 32 < K) {
-      const u32x4* src = reinterpret_cast<const u32x4*>(x + row * (size_t)K + (size_t)b * 32);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) in.q[i] = src[i];
+  const uint16_t* src = x + row * (size_t)K;
+  const int step = 1 << bits, first = lane & (step - 1);
+  bool bad = false;
+  auto load = [&](int i) {
+    u32x4 v = {0u, 0u, 0u, 0u};
+    if (i * 8 < K) v = *reinterpret_cast<const u32x4*>(src + (size_t)i * 8);
+    return v;
+  };
+  auto store = [&](int i, uint32_t codes, uint32_t sb) {
+    codes = fp4x8_to_ocp_doubled(codes);
+    const uint32_t st = sb == 0xFFu ? 127u : sb - 1u;
+    bad = bad || st < kScaleLo || st > kScaleHi;
+    // 8 bytes per lane: the codes of lanes 0, 1 | of lanes 2, 3 | the scale byte | zeros
+    uint32_t w0 = (uint32_t)__builtin_amdgcn_mov_dpp((int)codes, 0x08, 0xF, 0xF, true);  // of lanes 0, 2
+    uint32_t w1 = (uint32_t)__builtin_amdgcn_mov_dpp((int)codes, 0x0D, 0xF, 0xF, true);  // of lanes 1, 3
+    if ((i & 2) != 0) {
+      w0 = (i & 1) == 0 ? st : 0u;
+      w1 = 0u;
     }
-    uint32_t sb, codes[4];
-    quant_group32(in.d, sb, codes);
-    uint32_t st = 127u;
-    if (sb != 0xFFu) {
-      st = sb - 1u;
-      if (st < kScaleLo || st > kScaleHi) bad = 1;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) codes[j] = fp4x8_to_ocp_doubled(codes[j]);
-    }
-    uint8_t* blk = qrow + (size_t)b * 32;
-    *reinterpret_cast<u32x4*>(blk) = u32x4{codes[0], codes[1], codes[2], codes[3]};
-    *reinterpret_cast<u32x4*>(blk + 16) = u32x4{st, 0u, 0u, 0u};
-  }
-  bad = __syncthreads_or(bad);
-  if (threadIdx.x == 0) row_bad[row] = (uint8_t)(bad != 0);
+    *reinterpret_cast<u32x2*>(qrow + (size_t)(i >> 2) * 32 + (i & 3) * 8) = u32x2{w0, w1};
+  };
+  quant_row(first, step, pieces, load, store);
+  // the row's lanes are `step` consecutive ones (all of them here, or none: a row's lanes leave together)
+  const unsigned long long any = __ballot(bad);
+  const unsigned long long mine = (step == 64 ? ~0ull : ((1ull << step) - 1ull) << (lane & ~(step - 1)));
+  if (first == 0) row_bad[row] = (uint8_t)((any & mine) != 0ull);
 }
 
 // ---------------------------------------------------------------------------
@@ -1175,7 +1317,7 @@ bool mx_plan(const FusedMoeArgs& a, bool need_stage0, MxPlan& pl) {
 
 void mx_stage0(const FusedMoeArgs& a, const MxPlan& pl, hipStream_t stream) {
   if (pl.terms0 == 1) {
-    hipLaunchKernelGGL(quant_rows_w4_kernel, dim3(a.M), dim3(256), 0, stream, a.A, pl.aq, pl.abad, a.hidden, nullptr, 0, nullptr, 0);
+    hipLaunchKernelGGL(quant_rows_w4_kernel, quant_grid(a.M, mx_kp(a.hidden) / 8), dim3(256), 0, stream, a.A, pl.aq, pl.abad, a.hidden, a.M, nullptr, 0, nullptr, 0);
     launch_mx_stage_t<0, 1>(pl.g0, stream);
   } else if (pl.terms0 == 2) {
     hipLaunchKernelGGL(split_rows_fp6_kernel<2>, split_grid(a.M, a.hidden), dim3(256), 0, stream, a.A, pl.aq, pl.abad, a.hidden, a.hidden, a.M, nullptr, 0, nullptr, 0);
@@ -1190,7 +1332,7 @@ void mx_stage0(const FusedMoeArgs& a, const MxPlan& pl, hipStream_t stream) {
 // sorted positions) -> second stage -> per-token sum
 void mx_stage1(const FusedMoeArgs& a, const MxPlan& pl, hipStream_t stream) {
   if (pl.terms1 == 1) {
-    hipLaunchKernelGGL(quant_rows_w4_kernel, dim3(a.EM), dim3(256), 0, stream, a.act, pl.cq, pl.cbad, a.ispp, a.sorted_ids, a.M * a.top_k, pl.pos, a.M * a.top_k);
+    hipLaunchKernelGGL(quant_rows_w4_kernel, quant_grid(a.EM, mx_kp(a.ispp) / 8), dim3(256), 0, stream, a.act, pl.cq, pl.cbad, a.ispp, a.EM, a.sorted_ids, a.M * a.top_k, pl.pos, a.M * a.top_k);
     launch_mx_stage_t<1, 1>(pl.g1, stream);
   } else if (pl.terms1 == 2) {
     hipLaunchKernelGGL(split_rows_fp6_kernel<2>, split_grid(a.EM, a.ispp), dim3(256), 0, stream, a.act, pl.cq, pl.cbad, a.ispp, a.ispp, a.EM, a.sorted_ids, a.M * a.top_k, pl.pos, a.M * a.top_k);
@@ -1313,8 +1455,8 @@ void launch_split_rows_fp6(const uint16_t* x, int rows, int K, int terms, uint8_
 void launch_mxfp4_quant(const uint16_t* A, const int32_t* sorted_ids, uint8_t* packed, uint8_t* scales,
                         int rows, int hidden, int top_k, int n_flat, hipStream_t stream) {
   if (rows <= 0 || hidden <= 0) return;
-  hipLaunchKernelGGL(mxfp4_quant_kernel, dim3(rows), dim3(256), 0, stream, A, sorted_ids, packed, scales,
-                     hidden, top_k, n_flat);
+  hipLaunchKernelGGL(mxfp4_quant_kernel, quant_grid(rows, hidden / 8), dim3(256), 0, stream, A, sorted_ids,
+                     packed, scales, hidden, rows, top_k, n_flat);
 }
 
 }  // namespace vk
