@@ -46,7 +46,11 @@ __global__ __launch_bounds__(256) void act_epilogue_kernel(
   }
 }
 
-// pos[flat] = sorted row of every routed flat index (the others keep their -1).
+// pos[flat] = sorted row of every routed flat index.  The entries of the others hold
+// whatever the caller's workspace held: the combines take an entry only when sorted_ids says
+// that its row is that flat index's (routed_row), which saves the launch that would clear the
+// table (4.7 us and the gap before it, of 215 us for the orchestration ops around 4096 tokens
+// of 4096 and of 298 us for a tensor-parallel rank's share of 2048).
 __global__ __launch_bounds__(256) void invert_sorted_ids_kernel(const int32_t* __restrict__ sorted_ids,
                                                                 int32_t* __restrict__ pos, int EM,
                                                                 int n_flat) {
@@ -56,6 +60,35 @@ __global__ __launch_bounds__(256) void invert_sorted_ids_kernel(const int32_t* _
   if (flat >= 0 && flat < n_flat) pos[flat] = r;
 }
 
+// The sorted row of flat index `flat`, or -1 when it has none (uniform per workgroup).
+__device__ __forceinline__ int routed_row(const int32_t* __restrict__ pos,
+                                          const int32_t* __restrict__ sorted_ids, int flat, int EM) {
+  const int r = pos[flat];
+  return (unsigned)r < (unsigned)EM && sorted_ids[r] == flat ? r : -1;
+}
+
+// The token's sorted rows in ascending order, -1 (none) last: rows[0 .. TOPK).  Known at
+// compile time how many, they stay in scalar registers and the loads of all rows are
+// issued together; the order is an odd-even exchange over them.
+template <int TOPK>
+__device__ __forceinline__ void sorted_rows(const int32_t* __restrict__ pos,
+                                            const int32_t* __restrict__ sorted_ids, int t, int EM,
+                                            int (&rows)[TOPK]) {
+  unsigned key[TOPK];  // (as unsigned, -1 is the largest)
+#pragma unroll
+  for (int j = 0; j < TOPK; ++j) key[j] = (unsigned)routed_row(pos, sorted_ids, t * TOPK + j, EM);
+#pragma unroll
+  for (int i = 0; i < TOPK; ++i)
+#pragma unroll
+    for (int j = i & 1; j + 1 < TOPK; j += 2) {
+      const unsigned lo = min(key[j], key[j + 1]), hi = max(key[j], key[j + 1]);
+      key[j] = lo;
+      key[j + 1] = hi;
+    }
+#pragma unroll
+  for (int j = 0; j < TOPK; ++j) rows[j] = (int)key[j];
+}
+
 // Routed combine in gather form: out[t, :] += (partial[r, :] + bias[e(r), :]) * w[r] over
 // the token's sorted rows r in ascending order, which is the order the reference's loops
 // over the rows add them in (moe_combine_cpu, moe_fused.cpp:523-564; without a bias,
@@ -63,28 +96,22 @@ __global__ __launch_bounds__(256) void invert_sorted_ids_kernel(const int32_t* _
 // the sum into out are each rounded on their own, as there, so the result is the
 // reference's bit for bit.  A row of a block without an expert (expert_ids given) adds
 // nothing.  One thread per 4 columns.
+template <int TOPK>  // experts per token, 0 = any number (the next row looked for one at a time)
 __global__ __launch_bounds__(256) void combine_rows_kernel(
     const float* __restrict__ partial, const float* __restrict__ bias, const float* __restrict__ w_sorted,
-    const int32_t* __restrict__ pos, const int32_t* __restrict__ expert_ids, float* __restrict__ out,
-    int M, int width, int top_k, int block_size) {
+    const int32_t* __restrict__ pos, const int32_t* __restrict__ sorted_ids,
+    const int32_t* __restrict__ expert_ids, float* __restrict__ out, int M, int width, int top_k, int EM,
+    int block_size) {
   const int c = (blockIdx.x * blockDim.x + threadIdx.x) * 4;
   if (c >= width) return;
   for (int t = blockIdx.y; t < M; t += gridDim.y) {
     f32x4u* o = reinterpret_cast<f32x4u*>(out + (size_t)t * (size_t)width + c);
     f32x4 sum = *o;
-    int last = -1;
-    for (int s = 0; s < top_k; ++s) {   // the next larger sorted row of this token (top_k is small)
-      int r = 0x7FFFFFFF;
-      for (int j = 0; j < top_k; ++j) {
-        const int rj = pos[t * top_k + j];
-        if (rj > last && rj < r) r = rj;
-      }
-      if (r == 0x7FFFFFFF) break;
-      last = r;
+    auto load = [&](int r) { return *reinterpret_cast<const f32x4u*>(partial + (size_t)r * (size_t)width + c); };
+    auto add = [&](f32x4 p, int r) {
       int e = 0;
       if (expert_ids != nullptr) e = expert_ids[r / block_size];
-      if (e < 0) continue;
-      f32x4 p = *reinterpret_cast<const f32x4u*>(partial + (size_t)r * (size_t)width + c);
+      if (e < 0) return;
       if (bias != nullptr) p += *reinterpret_cast<const f32x4u*>(bias + (size_t)e * (size_t)width + c);
       const float w = w_sorted[r];
 #pragma unroll
@@ -92,6 +119,28 @@ __global__ __launch_bounds__(256) void combine_rows_kernel(
         float prod = p[i] * w;
         asm volatile("" : "+v"(prod));   // the rounded product is a value of its own: no fused multiply-add
         sum[i] += prod;
+      }
+    };
+    if constexpr (TOPK > 0) {
+      int rows[TOPK];
+      sorted_rows<TOPK>(pos, sorted_ids, t, EM, rows);
+      f32x4 p[TOPK];
+#pragma unroll
+      for (int s = 0; s < TOPK; ++s) p[s] = load(rows[s] < 0 ? 0 : rows[s]);
+#pragma unroll
+      for (int s = 0; s < TOPK; ++s)
+        if (rows[s] >= 0) add(p[s], rows[s]);
+    } else {
+      int last = -1;
+      for (int s = 0; s < top_k; ++s) {   // the next larger sorted row of this token (top_k is small)
+        int r = 0x7FFFFFFF;
+        for (int j = 0; j < top_k; ++j) {
+          const int rj = routed_row(pos, sorted_ids, t * top_k + j, EM);
+          if (rj > last && rj < r) r = rj;
+        }
+        if (r == 0x7FFFFFFF) break;
+        last = r;
+        add(load(r), r);
       }
     }
     *o = sum;
@@ -131,8 +180,8 @@ __global__ __launch_bounds__(256) void gather_rows_kernel(const uint8_t* __restr
 // form over the table of sorted positions; one thread per 8 columns (4 bytes of codes).
 __global__ __launch_bounds__(256) void combine_rows_q_kernel(
     const uint8_t* __restrict__ partial_q, const uint8_t* __restrict__ partial_s,
-    const float* __restrict__ w_sorted, const int32_t* __restrict__ pos, float* __restrict__ out, int M,
-    int width, int top_k) {
+    const float* __restrict__ w_sorted, const int32_t* __restrict__ pos,
+    const int32_t* __restrict__ sorted_ids, float* __restrict__ out, int M, int width, int top_k, int EM) {
   const int c = (blockIdx.x * blockDim.x + threadIdx.x) * 8;
   if (c >= width) return;
   const int groups = width / 32;
@@ -145,7 +194,7 @@ __global__ __launch_bounds__(256) void combine_rows_q_kernel(
     for (int s = 0; s < top_k; ++s) {   // the next larger sorted row of this token (top_k is small)
       int r = 0x7FFFFFFF;
       for (int j = 0; j < top_k; ++j) {
-        const int rj = pos[t * top_k + j];
+        const int rj = routed_row(pos, sorted_ids, t * top_k + j, EM);
         if (rj > last && rj < r) r = rj;
       }
       if (r == 0x7FFFFFFF) break;
@@ -189,12 +238,11 @@ void launch_mxfp4_scatter_reduce_q(const uint8_t* partial_q, const uint8_t* part
                                    const int32_t* sorted_ids, float* out, int M, int width, int top_k,
                                    int EM, int32_t* pos, hipStream_t stream) {
   if (M <= 0 || width <= 0 || EM <= 0) return;
-  launch_fill_i32(pos, -1, M * top_k, stream);
   hipLaunchKernelGGL(invert_sorted_ids_kernel, dim3((unsigned)((EM + 255) / 256)), dim3(256), 0, stream,
                      sorted_ids, pos, EM, M * top_k);
   const dim3 grid((unsigned)((width / 8 + 255) / 256), (unsigned)(M < 65535 ? M : 65535));
   hipLaunchKernelGGL(combine_rows_q_kernel, grid, dim3(256), 0, stream, partial_q, partial_s, topk_w, pos,
-                     out, M, width, top_k);
+                     sorted_ids, out, M, width, top_k, EM);
 }
 
 void launch_moe_act_epilogue(const float* gate_up, const float* b13, uint16_t* act,
@@ -213,12 +261,22 @@ void launch_moe_combine_sorted(const float* partial, const float* bias, const fl
                                int width, int top_k, int EM, int block_size, int32_t* pos,
                                hipStream_t stream) {
   if (M <= 0 || width <= 0 || EM <= 0) return;
-  launch_fill_i32(pos, -1, M * top_k, stream);
   hipLaunchKernelGGL(invert_sorted_ids_kernel, dim3((unsigned)((EM + 255) / 256)), dim3(256), 0, stream,
                      sorted_ids, pos, EM, M * top_k);
   const dim3 grid((unsigned)((width / 4 + 255) / 256), (unsigned)(M < 65535 ? M : 65535));
-  hipLaunchKernelGGL(combine_rows_kernel, grid, dim3(256), 0, stream, partial, bias, w_sorted, pos,
-                     expert_ids, out, M, width, top_k, block_size > 0 ? block_size : 16);
+  const int bs = block_size > 0 ? block_size : 16;
+  switch (top_k) {
+#define VK_COMBINE(K_)                                                                                   \
+  case K_:                                                                                               \
+    hipLaunchKernelGGL(combine_rows_kernel<K_>, grid, dim3(256), 0, stream, partial, bias, w_sorted, pos, \
+                       sorted_ids, expert_ids, out, M, width, top_k, EM, bs);                            \
+    break;
+    VK_COMBINE(1) VK_COMBINE(2) VK_COMBINE(4) VK_COMBINE(6) VK_COMBINE(8)
+#undef VK_COMBINE
+    default:
+      hipLaunchKernelGGL(combine_rows_kernel<0>, grid, dim3(256), 0, stream, partial, bias, w_sorted, pos,
+                         sorted_ids, expert_ids, out, M, width, top_k, EM, bs);
+  }
 }
 
 void launch_mxfp4_scatter_reduce(const float* partial, const float* topk_w, const int32_t* sorted_ids,
