@@ -120,6 +120,35 @@ def test_router_matches_oracle_bitwise(hip_lib):
         assert np.array_equal(w.cpu().numpy().view(np.uint32), rw.view(np.uint32)), (T, E, k)
 
 
+@pytest.mark.parametrize("M,k,E,share", [(1024, 8, 8, 1.0), (1025, 8, 8, 1.0), (8193, 1, 16, 0.99),
+                                         (16384, 8, 256, 0.0), (16384, 8, 4096, 0.07), (2047, 5, 4097, 0.5),
+                                         (4095, 3, 64, 0.33)])
+@pytest.mark.parametrize("with_map", [False, True])
+def test_align_lists_at_their_edges(hip_lib, M, k, E, share, with_map):
+    """A wavefront's list of matches full to the last entry (512 of a slice of 512), one
+    slice longer, past it, not there at all (more than 4096 experts), ragged last chunks."""
+    fn = ve.resolve_align_fn(hip_lib)
+    rng = np.random.default_rng(M * 31 + E)
+    N, bs = M * k, 16
+    ids = rng.integers(0, E, N).astype(np.int32)
+    ids[rng.random(N) < share] = E // 2
+    emap = rng.permutation(E).astype(np.int32) if with_map else None
+    max_em = ve._align_em_bound(M, k, E, bs)
+    d_ids = to_dev(ids)
+    d_map = None if emap is None else to_dev(emap)
+    sids = torch.full((max_em,), -7, dtype=torch.int32, device=dev())
+    eids = torch.full((max_em // bs,), -7, dtype=torch.int32, device=dev())
+    out_em = torch.full((1,), -7, dtype=torch.int32, device=dev())
+    st = fn(d_ids.data_ptr(), None if d_map is None else d_map.data_ptr(), M, k, bs, E, E, max_em,
+            sids.data_ptr(), eids.data_ptr(), out_em.data_ptr(), None)
+    assert st == 0
+    torch.cuda.synchronize()
+    rs, re, rem = oracle.moe_align_block_size_with_map(ids, E, bs, emap, local_n=E, max_EM=max_em)
+    assert int(out_em.item()) == rem
+    assert np.array_equal(sids.cpu().numpy(), rs)
+    assert np.array_equal(eids.cpu().numpy(), re)
+
+
 def test_align_matches_oracle_bitwise(hip_lib):
     fn = ve.resolve_align_fn(hip_lib)
     rng = np.random.default_rng(0)

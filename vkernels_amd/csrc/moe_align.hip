@@ -16,14 +16,16 @@
 //      entries of expert e in its own contiguous slice of the indices;
 //   2. sums the padded counts of the experts before it (its first row) and
 //      of all experts (EM);
-//   3. walks its slices again and writes the matching flat indices in
-//      order, ranked with ballot + popcount;
+//   3. writes the matching flat indices in order: each wavefront kept those of
+//      its slice in LDS as it walked, ranked with ballot + popcount, and walks
+//      again only where they are more than its list holds;
 //   4. pads its last block, writes its expert_ids and its share of the
 //      sentinel tail [EM, max_EM).
 // The routing table is read from L2 by every workgroup, and every workgroup
-// builds the whole histogram; for the largest benchmark shape (N = 131072,
-// 256 experts) that is 256 x 512 KiB of L2 reads and 75 us, against a layer
-// that takes milliseconds.
+// builds the whole histogram, which makes it bound by the vector instructions
+// per index: one walk instead of two and no clamps inside a slice took
+// N = 131072 with 256 experts from 66 to 25 us, N = 49146 with 64 from 27 to
+// 13.5 us, N = 16384 with 128 from 14.3 to 10.7 us; N = 128 is the launch (5 us).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -48,6 +50,11 @@ constexpr int kRouteAlignMaxTokens = 16, kRouteAlignMaxRows = 1024, kRouteAlignM
 constexpr int kAlignThreads = 1024;
 constexpr int kAlignWaves = kAlignThreads / 64;
 constexpr int kAlignAhead = 8;  // chunks of 64 indices a lane has in flight
+// Matches of the workgroup's expert that a wavefront keeps from its one walk (a wavefront
+// with more walks its slice a second time): 32 KiB of LDS, 16 times the even share of 256
+// experts at N = 131072.
+constexpr int kAlignList = 512;
+constexpr int kAlignListMaxExperts = 4096;
 
 __device__ __forceinline__ int local_expert(int ge, const int32_t* expert_map,
                                             int num_experts, int local_n) {
@@ -69,20 +76,58 @@ __device__ __forceinline__ int block_sum(int v, int* red) {
   return t;
 }
 
+// One wavefront's walk over its slice [begin, end) of the flat indices, in chunks of 64:
+// use(flat index, local expert or -1) of every lane, chunk after chunk.  A lane asks for
+// kAlignAhead chunks before it uses the first (one load per trip makes the walk a chain of
+// round trips to L2); while all of them lie inside the slice they are one address and
+// immediate offsets, no clamp and no bounds check per chunk.
+template <bool MAP, class Use>
+__device__ __forceinline__ void walk_slice(const int32_t* topk_ids, const int32_t* __restrict__ expert_map,
+                                           int begin, int end, int num_experts, int local_n, int lane,
+                                           Use&& use) {
+  const int valid = MAP ? num_experts : min(num_experts, local_n);
+  auto local = [&](int ge) {
+    if (MAP) return local_expert(ge, expert_map, num_experts, local_n);
+    return (unsigned)ge < (unsigned)max(valid, 0) ? ge : -1;
+  };
+  int base0 = begin;
+  for (; base0 + 64 * kAlignAhead <= end; base0 += 64 * kAlignAhead) {
+    const int32_t* const ids = topk_ids + base0 + lane;
+    int ge[kAlignAhead];
+#pragma unroll
+    for (int u = 0; u < kAlignAhead; ++u) ge[u] = ids[64 * u];
+#pragma unroll
+    for (int u = 0; u < kAlignAhead; ++u) use(base0 + 64 * u + lane, local(ge[u]));
+  }
+  for (; base0 < end; base0 += 64 * kAlignAhead) {
+    int ge[kAlignAhead];
+#pragma unroll
+    for (int u = 0; u < kAlignAhead; ++u) ge[u] = topk_ids[min(base0 + 64 * u + lane, end - 1)];
+#pragma unroll
+    for (int u = 0; u < kAlignAhead; ++u) {
+      const int base = base0 + 64 * u;
+      if (base >= end) break;  // uniform
+      use(base + lane, base + lane < end ? local(ge[u]) : -1);
+    }
+  }
+}
+
 // The work of workgroup blockIdx.x (steps 1 to 4 above).  topk_ids: the N flat routing
-// indices, in global memory or in LDS; hist: local_n ints of LDS.
+// indices, in global memory or in LDS; hist: local_n ints of LDS, and list_cap more per
+// wavefront behind them for the matches of expert e.
+template <bool MAP>
 __device__ __forceinline__ void align_workgroup(
     const int32_t* topk_ids, const int32_t* __restrict__ expert_map,
     int N, int block_size, int num_experts, int local_n, int max_EM,
     int32_t* __restrict__ sorted_ids, int32_t* __restrict__ expert_ids,
-    int32_t* __restrict__ out_em, int32_t* hist) {
+    int32_t* __restrict__ out_em, int32_t* hist, int32_t* lists, int list_cap) {
   __shared__ int wave_cnt[kAlignWaves];
   __shared__ int red[kAlignWaves];
 
   const int e = blockIdx.x;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = tid >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
   for (int i = tid; i < local_n; i += kAlignThreads) hist[i] = 0;
   __syncthreads();
@@ -92,36 +137,30 @@ __device__ __forceinline__ void align_workgroup(
   const int slice = ((N + kAlignWaves - 1) / kAlignWaves + 63) & ~63;
   const int begin = wave * slice;
   const int end = min(N, begin + slice);
+  const unsigned long long lower = (1ull << lane) - 1ull;
 
-  // A lane asks for kAlignAhead chunks of 64 indices before it uses the first: one
-  // load per trip makes the walk a chain of round trips to L2 (two walks of N / 1024
-  // trips each; N = 131072, 256 experts: 92 us that way, 75 us this way).
   int mine = 0;
-  for (int base0 = begin; base0 < end; base0 += 64 * kAlignAhead) {
-    int ids_ahead[kAlignAhead];
-#pragma unroll
-    for (int u = 0; u < kAlignAhead; ++u) ids_ahead[u] = topk_ids[min(base0 + 64 * u + lane, end - 1)];
-#pragma unroll
-    for (int u = 0; u < kAlignAhead; ++u) {
-      const int base = base0 + 64 * u;
-      if (base >= end) break;  // uniform
-      const int i = base + lane;
-      const int le = i < end ? local_expert(ids_ahead[u], expert_map, num_experts, local_n) : -1;
-      if (le >= 0) {
-        // A wavefront whose lanes all hit one expert adds once instead of
-        // serialising 64 atomics on one address.
-        const int first = __builtin_amdgcn_readfirstlane(le);
-        const unsigned long long same = __ballot(le == first);
-        const unsigned long long active = __ballot(1);
-        if (same == active) {
-          if (lane == (int)__builtin_ctzll(active)) atomicAdd(&hist[first], (int)__popcll(active));
-        } else {
-          atomicAdd(&hist[le], 1);
-        }
+  int32_t* const list = lists + wave * list_cap;
+  walk_slice<MAP>(topk_ids, expert_map, begin, end, num_experts, local_n, lane, [&](int i, int le) {
+    if (le >= 0) {
+      // A wavefront whose lanes all hit one expert adds once instead of
+      // serialising 64 atomics on one address.
+      const int first = __builtin_amdgcn_readfirstlane(le);
+      const unsigned long long same = __ballot(le == first);
+      const unsigned long long active = __ballot(1);
+      if (same == active) {
+        if (lane == (int)__builtin_ctzll(active)) atomicAdd(&hist[first], (int)__popcll(active));
+      } else {
+        atomicAdd(&hist[le], 1);
       }
-      mine += (int)__popcll(__ballot(le == e));
     }
-  }
+    const unsigned long long match = __ballot(le == e);
+    if (match != 0ull) {  // uniform
+      const int at = mine + (int)__popcll(match & lower);
+      if (le == e && at < list_cap) list[at] = i;
+      mine += (int)__popcll(match);
+    }
+  });
   if (lane == 0) wave_cnt[wave] = mine;
   __syncthreads();
 
@@ -147,24 +186,20 @@ __device__ __forceinline__ void align_workgroup(
   for (int w = 0; w < wave; ++w) wave_base += wave_cnt[w];
 
   if (count > 0) {
-    int running = before + wave_base;
-    for (int base0 = begin; base0 < end; base0 += 64 * kAlignAhead) {
-      int ids_ahead[kAlignAhead];
-#pragma unroll
-      for (int u = 0; u < kAlignAhead; ++u) ids_ahead[u] = topk_ids[min(base0 + 64 * u + lane, end - 1)];
-#pragma unroll
-      for (int u = 0; u < kAlignAhead; ++u) {
-        const int base = base0 + 64 * u;
-        if (base >= end) break;  // uniform
-        const int i = base + lane;
-        const int le = i < end ? local_expert(ids_ahead[u], expert_map, num_experts, local_n) : -1;
+    const int row0 = before + wave_base;
+    if (mine <= list_cap) {  // uniform per wavefront: its own list, written by itself
+      for (int j = lane; j < mine; j += 64)
+        if (row0 + j < max_EM) sorted_ids[row0 + j] = list[j];
+    } else {
+      int running = row0;
+      walk_slice<MAP>(topk_ids, expert_map, begin, end, num_experts, local_n, lane, [&](int i, int le) {
         const unsigned long long match = __ballot(le == e);
         if (le == e) {
-          const int pos = running + (int)__popcll(match & ((1ull << lane) - 1ull));
+          const int pos = running + (int)__popcll(match & lower);
           if (pos < max_EM) sorted_ids[pos] = i;
         }
         running += (int)__popcll(match);
-      }
+      });
     }
     for (int r = before + count + tid; r < before + padded; r += kAlignThreads)
       if (r < max_EM) sorted_ids[r] = N;
@@ -189,14 +224,15 @@ __device__ __forceinline__ void align_workgroup(
   }
 }
 
+template <bool MAP>
 __global__ __launch_bounds__(kAlignThreads) void align_kernel(
     const int32_t* __restrict__ topk_ids, const int32_t* __restrict__ expert_map,
     int N, int block_size, int num_experts, int local_n, int max_EM,
     int32_t* __restrict__ sorted_ids, int32_t* __restrict__ expert_ids,
-    int32_t* __restrict__ out_em) {
-  extern __shared__ int32_t hist[];  // [local_n]
-  align_workgroup(topk_ids, expert_map, N, block_size, num_experts, local_n, max_EM, sorted_ids,
-                  expert_ids, out_em, hist);
+    int32_t* __restrict__ out_em, int list_cap) {
+  extern __shared__ int32_t lds[];  // [max(local_n, 1)] histogram, [kAlignWaves][list_cap] matches
+  align_workgroup<MAP>(topk_ids, expert_map, N, block_size, num_experts, local_n, max_EM, sorted_ids,
+                       expert_ids, out_em, lds, lds + (local_n > 0 ? local_n : 1), list_cap);
 }
 
 // Router and alignment in one launch, for decode-sized batches: every workgroup routes
@@ -212,7 +248,8 @@ __global__ __launch_bounds__(kAlignThreads) void route_align_kernel(
     int32_t* __restrict__ topk_ids, float* __restrict__ topk_w,
     int32_t* __restrict__ sorted_ids, int32_t* __restrict__ expert_ids,
     int32_t* __restrict__ out_em) {
-  extern __shared__ int32_t lds[];  // [max(local_n, 1)] histogram, [T * top_k] routing indices
+  // [max(local_n, 1)] histogram, [T * top_k] routing indices, [kAlignWaves][64] matches
+  extern __shared__ int32_t lds[];
   int32_t* const ids = lds + (local_n > 0 ? local_n : 1);
   const int lane = threadIdx.x & 63;
   for (int token = threadIdx.x >> 6; token < T; token += kAlignWaves) {  // uniform per wavefront
@@ -228,8 +265,14 @@ __global__ __launch_bounds__(kAlignThreads) void route_align_kernel(
     }
   }
   __syncthreads();
-  align_workgroup(ids, expert_map, T * top_k, block_size, E, local_n, max_EM, sorted_ids, expert_ids,
-                  out_em, lds);
+  // (a wavefront's slice is one chunk of 64: T * top_k <= kRouteAlignMaxRows)
+  int32_t* const lists = ids + T * top_k;
+  if (expert_map != nullptr)
+    align_workgroup<true>(ids, expert_map, T * top_k, block_size, E, local_n, max_EM, sorted_ids, expert_ids,
+                          out_em, lds, lists, 64);
+  else
+    align_workgroup<false>(ids, nullptr, T * top_k, block_size, E, local_n, max_EM, sorted_ids, expert_ids,
+                           out_em, lds, lists, 64);
 }
 
 }  // namespace
@@ -245,7 +288,7 @@ void launch_route_align(const float* logits, int T, int E, int top_k, int renorm
                         int32_t* topk_ids, float* topk_w, int32_t* sorted_ids, int32_t* expert_ids,
                         int32_t* out_em, hipStream_t stream) {
   const int groups = local_n > 0 ? local_n : 1;
-  const size_t lds = sizeof(int32_t) * ((size_t)groups + (size_t)T * (size_t)top_k);
+  const size_t lds = sizeof(int32_t) * ((size_t)groups + (size_t)T * (size_t)top_k + kAlignWaves * 64);
 #define VK_ROUTE_ALIGN_LAUNCH(PER)                                                                     \
   hipLaunchKernelGGL((route_align_kernel<PER>), dim3(groups), dim3(kAlignThreads), lds, stream, logits, \
                      T, E, top_k, renormalize, expert_map, block_size, local_n, max_EM, topk_ids,       \
@@ -264,10 +307,16 @@ void launch_align(const int32_t* topk_ids, const int32_t* expert_map, int N,
                   hipStream_t stream) {
   // local_n == 0 still needs one workgroup to write the sentinels and EM.
   const int groups = local_n > 0 ? local_n : 1;
-  const size_t lds = sizeof(int32_t) * (size_t)(local_n > 0 ? local_n : 1);
-  hipLaunchKernelGGL(align_kernel, dim3(groups), dim3(kAlignThreads), lds, stream,
-                     topk_ids, expert_map, N, block_size, num_experts, local_n,
-                     max_EM, sorted_ids, expert_ids, out_em);
+  // The lists take what the histogram leaves of 48 KiB, so that no number of experts that
+  // the histogram alone has room for is refused; none means a second walk, as before.
+  const int list_cap = local_n <= kAlignListMaxExperts ? kAlignList : 0;
+  const size_t lds = sizeof(int32_t) * ((size_t)groups + (size_t)list_cap * kAlignWaves);
+  if (expert_map != nullptr)
+    hipLaunchKernelGGL(align_kernel<true>, dim3(groups), dim3(kAlignThreads), lds, stream, topk_ids, expert_map,
+                       N, block_size, num_experts, local_n, max_EM, sorted_ids, expert_ids, out_em, list_cap);
+  else
+    hipLaunchKernelGGL(align_kernel<false>, dim3(groups), dim3(kAlignThreads), lds, stream, topk_ids, expert_map,
+                       N, block_size, num_experts, local_n, max_EM, sorted_ids, expert_ids, out_em, list_cap);
 }
 
 }  // namespace vk
