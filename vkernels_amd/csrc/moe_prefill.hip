@@ -1081,7 +1081,7 @@ __global__ __launch_bounds__(64 * kMxWaves) void tile_mx_kernel(MxArgs p) {
         // A wavefront runs alone on its SIMD, so every branch and every predicate of this
         // code is paid in full; it is therefore specialised, per row tile, on what is
         // uniform: a bias or none, and whether the tile's 32 rows all belong to this
-        // workgroup's window.  Then rows that are not routed are stored like the others
+        // workgroup's window.  (Nontemporal stores: combine_kernel.)  Then rows that are not routed are stored like the others
         // (with a routing weight of zero): nothing reads them (pos never points at them),
         // and a later segment of this window, if they are its rows, overwrites them.
         constexpr int kPitch = kMxYPitch;
@@ -1114,9 +1114,10 @@ __global__ __launch_bounds__(64 * kMxWaves) void tile_mx_kernel(MxArgs p) {
 #pragma unroll
             for (int pass = 0; pass < 8; ++pass) {
               if constexpr (kGuard) {
-                if ((routed >> (pass * 4 + (lane >> 4))) & 1ull) *reinterpret_cast<f32x4*>(dst) = v[pass];
+                if ((routed >> (pass * 4 + (lane >> 4))) & 1ull)
+                  __builtin_nontemporal_store(v[pass], reinterpret_cast<f32x4*>(dst));
               } else {
-                *reinterpret_cast<f32x4*>(dst) = v[pass];
+                __builtin_nontemporal_store(v[pass], reinterpret_cast<f32x4*>(dst));
               }
               dst += 4 * (size_t)p.ncols;
             }

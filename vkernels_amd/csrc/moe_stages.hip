@@ -107,7 +107,9 @@ __global__ __launch_bounds__(256) void combine_rows_kernel(
   for (int t = blockIdx.y; t < M; t += gridDim.y) {
     f32x4u* o = reinterpret_cast<f32x4u*>(out + (size_t)t * (size_t)width + c);
     f32x4 sum = *o;
-    auto load = [&](int r) { return *reinterpret_cast<const f32x4u*>(partial + (size_t)r * (size_t)width + c); };
+    auto load = [&](int r) {
+      return __builtin_nontemporal_load(reinterpret_cast<const f32x4u*>(partial + (size_t)r * (size_t)width + c));
+    };
     auto add = [&](f32x4 p, int r) {
       int e = 0;
       if (expert_ids != nullptr) e = expert_ids[r / block_size];
