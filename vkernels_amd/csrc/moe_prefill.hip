@@ -978,6 +978,7 @@ __global__ __launch_bounds__(64 * kMxWaves) void tile_mx_kernel(MxArgs p) {
       if constexpr (PREACT) {
         // the accumulators as they are: 64 columns (two tiles) at a time through the
         // wavefront's staging area, whole lines out, routed rows only
+        // (nontemporal: read once, by the activation or the combine)
         constexpr int kPitch = kMxYPitch;
         const int width = STAGE == 0 ? 2 * p.ncols : p.ncols;
 #pragma unroll
@@ -1003,7 +1004,8 @@ __global__ __launch_bounds__(64 * kMxWaves) void tile_mx_kernel(MxArgs p) {
           float* dst = p.preact + (size_t)(row0 + m * 32 + (lane >> 4)) * (size_t)width + col0 + (lane & 15) * 4;
 #pragma unroll
           for (int pass = 0; pass < 8; ++pass) {
-            if ((routed >> (pass * 4 + (lane >> 4))) & 1ull) *reinterpret_cast<f32x4*>(dst) = v[pass];
+            if ((routed >> (pass * 4 + (lane >> 4))) & 1ull)
+              __builtin_nontemporal_store(v[pass], reinterpret_cast<f32x4*>(dst));
             dst += 4 * (size_t)width;
           }
         }

@@ -18,7 +18,8 @@ namespace {
 // act[r, c] = bf16(activation(gate_up[r, c] + b13[e, c], gate_up[r, ispp + c] + b13[e, ispp + c]))
 // for every routed sorted row r of a block with an expert (moe_act_epilogue_cpu,
 // src/c/vkernels/kernels/moe_fused.cpp:370-422); the other rows of act are left as they
-// are.  One thread per 4 columns.
+// are.  One thread per 4 columns.  The pre-activations are read once, past the caches (with the
+// stage kernels' stores of them: a rank of four's share of 2048 tokens 266.8 -> 262.6 us).
 __global__ __launch_bounds__(256) void act_epilogue_kernel(
     const float* __restrict__ gate_up, const float* __restrict__ b13, uint16_t* __restrict__ act,
     const int32_t* __restrict__ sorted_ids, const int32_t* __restrict__ expert_ids, int n_flat, int EM,
@@ -30,8 +31,8 @@ __global__ __launch_bounds__(256) void act_epilogue_kernel(
     const int e = expert_ids[r / block_size];
     if (flat < 0 || flat >= n_flat || e < 0) continue;
     const float* row = gate_up + (size_t)r * (size_t)(2 * ispp);
-    f32x4 g = *reinterpret_cast<const f32x4*>(row + c);
-    f32x4 u = *reinterpret_cast<const f32x4*>(row + ispp + c);
+    f32x4 g = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(row + c));
+    f32x4 u = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(row + ispp + c));
     if (b13 != nullptr) {
       const float* b = b13 + (size_t)e * (size_t)(2 * ispp);
       g += *reinterpret_cast<const f32x4u*>(b + c);
