@@ -121,12 +121,12 @@ def test_router_matches_oracle_bitwise(hip_lib):
 
 
 @pytest.mark.parametrize("M,k,E,share", [(1024, 8, 8, 1.0), (1025, 8, 8, 1.0), (8193, 1, 16, 0.99),
-                                         (16384, 8, 256, 0.0), (16384, 8, 4096, 0.07), (2047, 5, 4097, 0.5),
+                                         (16384, 8, 256, 0.0), (16384, 8, 1024, 0.07), (2047, 5, 1024 - 1, 0.5),
                                          (4095, 3, 64, 0.33)])
 @pytest.mark.parametrize("with_map", [False, True])
 def test_align_lists_at_their_edges(hip_lib, M, k, E, share, with_map):
     """A wavefront's list of matches full to the last entry (512 of a slice of 512), one
-    slice longer, past it, not there at all (more than 4096 experts), ragged last chunks."""
+    slice longer, past it, as many experts as the call takes, ragged last chunks."""
     fn = ve.resolve_align_fn(hip_lib)
     rng = np.random.default_rng(M * 31 + E)
     N, bs = M * k, 16
