@@ -31,6 +31,7 @@
 
 #include "moe_route.hpp"
 #include "vk_internal.hpp"
+#include "vkernels_hip.h"
 
 // (the router's arithmetic is spelled out operation by operation: no contraction here)
 #pragma clang fp contract(off)
@@ -54,7 +55,8 @@ constexpr int kAlignAhead = 8;  // chunks of 64 indices a lane has in flight
 // with more walks its slice a second time): 32 KiB of LDS, 16 times the even share of 256
 // experts at N = 131072.
 constexpr int kAlignList = 512;
-constexpr int kAlignListMaxExperts = 4096;
+static_assert(sizeof(int32_t) * (VK_HIP_ALIGN_MAX_EXPERTS + kAlignWaves * kAlignList) <= 48 * 1024,
+              "histogram and lists within the LDS a launch has without asking for more");
 
 __device__ __forceinline__ int local_expert(int ge, const int32_t* expert_map,
                                             int num_experts, int local_n) {
@@ -113,14 +115,14 @@ __device__ __forceinline__ void walk_slice(const int32_t* topk_ids, const int32_
 }
 
 // The work of workgroup blockIdx.x (steps 1 to 4 above).  topk_ids: the N flat routing
-// indices, in global memory or in LDS; hist: local_n ints of LDS, and list_cap more per
-// wavefront behind them for the matches of expert e.
-template <bool MAP>
+// indices, in global memory or in LDS; hist: local_n ints of LDS; lists: LIST more per
+// wavefront for the matches of expert e.
+template <bool MAP, int LIST>
 __device__ __forceinline__ void align_workgroup(
     const int32_t* topk_ids, const int32_t* __restrict__ expert_map,
     int N, int block_size, int num_experts, int local_n, int max_EM,
     int32_t* __restrict__ sorted_ids, int32_t* __restrict__ expert_ids,
-    int32_t* __restrict__ out_em, int32_t* hist, int32_t* lists, int list_cap) {
+    int32_t* __restrict__ out_em, int32_t* hist, int32_t* lists) {
   __shared__ int wave_cnt[kAlignWaves];
   __shared__ int red[kAlignWaves];
 
@@ -140,7 +142,7 @@ __device__ __forceinline__ void align_workgroup(
   const unsigned long long lower = (1ull << lane) - 1ull;
 
   int mine = 0;
-  int32_t* const list = lists + wave * list_cap;
+  int32_t* const list = lists + wave * LIST;
   walk_slice<MAP>(topk_ids, expert_map, begin, end, num_experts, local_n, lane, [&](int i, int le) {
     if (le >= 0) {
       // A wavefront whose lanes all hit one expert adds once instead of
@@ -157,7 +159,7 @@ __device__ __forceinline__ void align_workgroup(
     const unsigned long long match = __ballot(le == e);
     if (match != 0ull) {  // uniform
       const int at = mine + (int)__popcll(match & lower);
-      if (le == e && at < list_cap) list[at] = i;
+      if (le == e && at < LIST) list[at] = i;
       mine += (int)__popcll(match);
     }
   });
@@ -187,7 +189,7 @@ __device__ __forceinline__ void align_workgroup(
 
   if (count > 0) {
     const int row0 = before + wave_base;
-    if (mine <= list_cap) {  // uniform per wavefront: its own list, written by itself
+    if (mine <= LIST) {  // uniform per wavefront: its own list, written by itself
       for (int j = lane; j < mine; j += 64)
         if (row0 + j < max_EM) sorted_ids[row0 + j] = list[j];
     } else {
@@ -229,10 +231,10 @@ __global__ __launch_bounds__(kAlignThreads) void align_kernel(
     const int32_t* __restrict__ topk_ids, const int32_t* __restrict__ expert_map,
     int N, int block_size, int num_experts, int local_n, int max_EM,
     int32_t* __restrict__ sorted_ids, int32_t* __restrict__ expert_ids,
-    int32_t* __restrict__ out_em, int list_cap) {
-  extern __shared__ int32_t lds[];  // [max(local_n, 1)] histogram, [kAlignWaves][list_cap] matches
-  align_workgroup<MAP>(topk_ids, expert_map, N, block_size, num_experts, local_n, max_EM, sorted_ids,
-                       expert_ids, out_em, lds, lds + (local_n > 0 ? local_n : 1), list_cap);
+    int32_t* __restrict__ out_em) {
+  extern __shared__ int32_t lds[];  // [max(local_n, 1)] histogram, [kAlignWaves][kAlignList] matches
+  align_workgroup<MAP, kAlignList>(topk_ids, expert_map, N, block_size, num_experts, local_n, max_EM,
+                                   sorted_ids, expert_ids, out_em, lds, lds + (local_n > 0 ? local_n : 1));
 }
 
 // Router and alignment in one launch, for decode-sized batches: every workgroup routes
@@ -268,11 +270,11 @@ __global__ __launch_bounds__(kAlignThreads) void route_align_kernel(
   // (a wavefront's slice is one chunk of 64: T * top_k <= kRouteAlignMaxRows)
   int32_t* const lists = ids + T * top_k;
   if (expert_map != nullptr)
-    align_workgroup<true>(ids, expert_map, T * top_k, block_size, E, local_n, max_EM, sorted_ids, expert_ids,
-                          out_em, lds, lists, 64);
+    align_workgroup<true, 64>(ids, expert_map, T * top_k, block_size, E, local_n, max_EM, sorted_ids,
+                              expert_ids, out_em, lds, lists);
   else
-    align_workgroup<false>(ids, nullptr, T * top_k, block_size, E, local_n, max_EM, sorted_ids, expert_ids,
-                           out_em, lds, lists, 64);
+    align_workgroup<false, 64>(ids, nullptr, T * top_k, block_size, E, local_n, max_EM, sorted_ids, expert_ids,
+                               out_em, lds, lists);
 }
 
 }  // namespace
@@ -307,16 +309,13 @@ void launch_align(const int32_t* topk_ids, const int32_t* expert_map, int N,
                   hipStream_t stream) {
   // local_n == 0 still needs one workgroup to write the sentinels and EM.
   const int groups = local_n > 0 ? local_n : 1;
-  // The lists take what the histogram leaves of 48 KiB, so that no number of experts that
-  // the histogram alone has room for is refused; none means a second walk, as before.
-  const int list_cap = local_n <= kAlignListMaxExperts ? kAlignList : 0;
-  const size_t lds = sizeof(int32_t) * ((size_t)groups + (size_t)list_cap * kAlignWaves);
+  const size_t lds = sizeof(int32_t) * ((size_t)groups + (size_t)kAlignList * kAlignWaves);
   if (expert_map != nullptr)
     hipLaunchKernelGGL(align_kernel<true>, dim3(groups), dim3(kAlignThreads), lds, stream, topk_ids, expert_map,
-                       N, block_size, num_experts, local_n, max_EM, sorted_ids, expert_ids, out_em, list_cap);
+                       N, block_size, num_experts, local_n, max_EM, sorted_ids, expert_ids, out_em);
   else
     hipLaunchKernelGGL(align_kernel<false>, dim3(groups), dim3(kAlignThreads), lds, stream, topk_ids, expert_map,
-                       N, block_size, num_experts, local_n, max_EM, sorted_ids, expert_ids, out_em, list_cap);
+                       N, block_size, num_experts, local_n, max_EM, sorted_ids, expert_ids, out_em);
 }
 
 }  // namespace vk
