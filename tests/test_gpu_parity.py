@@ -149,6 +149,37 @@ def test_align_lists_at_their_edges(hip_lib, M, k, E, share, with_map):
     assert np.array_equal(eids.cpu().numpy(), re)
 
 
+@pytest.mark.parametrize("N", [1, 63, 64, 65, 960, 1023, 1024, 1025])
+@pytest.mark.parametrize("with_map", [False, True])
+def test_align_an_index_per_lane_at_its_edges(hip_lib, N, with_map):
+    """Around full wavefronts and around the most indices that stay in registers; indices out
+    of range, experts of another rank, an expert with most of them, and a caller's max_EM that
+    is too short for the rows (out_EM is then max_EM, and nothing is written beyond)."""
+    fn = ve.resolve_align_fn(hip_lib)
+    rng = np.random.default_rng(N)
+    for E, bs, hot, cut in ((1, 16, 0.0, False), (37, 16, 0.7, False), (1024, 32, 0.0, False), (64, 16, 0.3, True)):
+        ids = rng.integers(-2, E + 2, N).astype(np.int32)
+        ids[rng.random(N) < hot] = E // 3
+        emap, local_n = None, E
+        if with_map:
+            local_n = max(1, E // 2)
+            emap = np.full(E, -1, np.int32)
+            emap[rng.permutation(E)[:local_n]] = np.arange(local_n, dtype=np.int32)
+        max_em = bs * max(1, N // (2 * bs)) if cut else ve._align_em_bound(N, 1, local_n, bs)
+        d_ids, d_map = to_dev(ids), None if emap is None else to_dev(emap)
+        sids = torch.full((max_em + 8,), -7, dtype=torch.int32, device=dev())
+        eids = torch.full((max_em // bs + 8,), -7, dtype=torch.int32, device=dev())
+        out_em = torch.full((1,), -7, dtype=torch.int32, device=dev())
+        assert fn(d_ids.data_ptr(), None if d_map is None else d_map.data_ptr(), N, 1, bs, E, local_n, max_em,
+                  sids.data_ptr(), eids.data_ptr(), out_em.data_ptr(), None) == 0
+        torch.cuda.synchronize()
+        whole = ve._align_em_bound(N, 1, local_n, bs)
+        rs, re, rem = oracle.moe_align_block_size_with_map(ids, E, bs, emap, local_n=local_n, max_EM=whole)
+        assert int(out_em.item()) == min(rem, max_em)
+        assert np.array_equal(sids.cpu().numpy(), np.r_[rs[:max_em], np.full(8, -7)])
+        assert np.array_equal(eids.cpu().numpy(), np.r_[re[:max_em // bs], np.full(8, -7)])
+
+
 def test_align_matches_oracle_bitwise(hip_lib):
     fn = ve.resolve_align_fn(hip_lib)
     rng = np.random.default_rng(0)

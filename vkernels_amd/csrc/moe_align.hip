@@ -18,14 +18,16 @@
 //      of all experts (EM);
 //   3. writes the matching flat indices in order: each wavefront kept those of
 //      its slice in LDS as it walked, ranked with ballot + popcount, and walks
-//      again only where they are more than its list holds;
+//      again only where they are more than its list holds (up to 1024 indices
+//      there is no walk: a lane holds one);
 //   4. pads its last block, writes its expert_ids and its share of the
 //      sentinel tail [EM, max_EM).
 // The routing table is read from L2 by every workgroup, and every workgroup
 // builds the whole histogram, which makes it bound by the vector instructions
 // per index: one walk instead of two and no clamps inside a slice took
-// N = 131072 with 256 experts from 66 to 25 us, N = 49146 with 64 from 27 to
-// 13.5 us, N = 16384 with 128 from 14.3 to 10.7 us; N = 128 is the launch (5 us).
+// N = 131072 with 256 experts from 61 to 21 us, N = 49146 with 64 from 26 to
+// 12.5 us, N = 16384 with 128 from 12.0 to 7.7 us.  Up to 1024 indices a lane
+// holds its index, and the launch is what the time is (4.6 to 5.8 us).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -55,6 +57,7 @@ constexpr int kAlignAhead = 8;  // chunks of 64 indices a lane has in flight
 // with more walks its slice a second time): 32 KiB of LDS, 16 times the even share of 256
 // experts at N = 131072.
 constexpr int kAlignList = 512;
+static_assert(kRouteAlignMaxRows <= kAlignThreads, "an index per lane");
 static_assert(sizeof(int32_t) * (VK_HIP_ALIGN_MAX_EXPERTS + kAlignWaves * kAlignList) <= 48 * 1024,
               "histogram and lists within the LDS a launch has without asking for more");
 
@@ -115,9 +118,10 @@ __device__ __forceinline__ void walk_slice(const int32_t* topk_ids, const int32_
 }
 
 // The work of workgroup blockIdx.x (steps 1 to 4 above).  topk_ids: the N flat routing
-// indices, in global memory or in LDS; hist: local_n ints of LDS; lists: LIST more per
-// wavefront for the matches of expert e.
-template <bool MAP, int LIST>
+// indices, in global memory or in LDS; hist: local_n ints of LDS; lists: kAlignList more per
+// wavefront for the matches of expert e, unused with ONE.  ONE: N <= kAlignThreads, an index
+// per lane, which stays in its register: no list, no walk.
+template <bool MAP, bool ONE>
 __device__ __forceinline__ void align_workgroup(
     const int32_t* topk_ids, const int32_t* __restrict__ expert_map,
     int N, int block_size, int num_experts, int local_n, int max_EM,
@@ -131,19 +135,21 @@ __device__ __forceinline__ void align_workgroup(
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
+  int own = -1;  // ONE: the local expert of this lane's index
+  if constexpr (ONE)
+    if (tid < N) own = local_expert(topk_ids[tid], MAP ? expert_map : nullptr, num_experts, local_n);
+
   for (int i = tid; i < local_n; i += kAlignThreads) hist[i] = 0;
   __syncthreads();
 
   // Slice of the flat indices owned by this wavefront (a multiple of 64 long
   // so that every step of the walk is a full wavefront).
-  const int slice = ((N + kAlignWaves - 1) / kAlignWaves + 63) & ~63;
+  const int slice = ONE ? 64 : ((N + kAlignWaves - 1) / kAlignWaves + 63) & ~63;
   const int begin = wave * slice;
   const int end = min(N, begin + slice);
   const unsigned long long lower = (1ull << lane) - 1ull;
 
-  int mine = 0;
-  int32_t* const list = lists + wave * LIST;
-  walk_slice<MAP>(topk_ids, expert_map, begin, end, num_experts, local_n, lane, [&](int i, int le) {
+  auto histogram = [&](int le) {
     if (le >= 0) {
       // A wavefront whose lanes all hit one expert adds once instead of
       // serialising 64 atomics on one address.
@@ -156,13 +162,23 @@ __device__ __forceinline__ void align_workgroup(
         atomicAdd(&hist[le], 1);
       }
     }
-    const unsigned long long match = __ballot(le == e);
-    if (match != 0ull) {  // uniform
-      const int at = mine + (int)__popcll(match & lower);
-      if (le == e && at < LIST) list[at] = i;
-      mine += (int)__popcll(match);
-    }
-  });
+  };
+  int mine = 0;
+  int32_t* const list = lists + wave * kAlignList;
+  if constexpr (ONE) {
+    histogram(own);
+    mine = (int)__popcll(__ballot(own == e));
+  } else {
+    walk_slice<MAP>(topk_ids, expert_map, begin, end, num_experts, local_n, lane, [&](int i, int le) {
+      histogram(le);
+      const unsigned long long match = __ballot(le == e);
+      if (match != 0ull) {  // uniform
+        const int at = mine + (int)__popcll(match & lower);
+        if (le == e && at < kAlignList) list[at] = i;
+        mine += (int)__popcll(match);
+      }
+    });
+  }
   if (lane == 0) wave_cnt[wave] = mine;
   __syncthreads();
 
@@ -189,7 +205,10 @@ __device__ __forceinline__ void align_workgroup(
 
   if (count > 0) {
     const int row0 = before + wave_base;
-    if (mine <= LIST) {  // uniform per wavefront: its own list, written by itself
+    if constexpr (ONE) {
+      const int pos = row0 + (int)__popcll(__ballot(own == e) & lower);
+      if (own == e && pos < max_EM) sorted_ids[pos] = tid;
+    } else if (mine <= kAlignList) {  // uniform per wavefront: its own list, written by itself
       for (int j = lane; j < mine; j += 64)
         if (row0 + j < max_EM) sorted_ids[row0 + j] = list[j];
     } else {
@@ -226,15 +245,15 @@ __device__ __forceinline__ void align_workgroup(
   }
 }
 
-template <bool MAP>
+template <bool MAP, bool ONE>
 __global__ __launch_bounds__(kAlignThreads) void align_kernel(
     const int32_t* __restrict__ topk_ids, const int32_t* __restrict__ expert_map,
     int N, int block_size, int num_experts, int local_n, int max_EM,
     int32_t* __restrict__ sorted_ids, int32_t* __restrict__ expert_ids,
     int32_t* __restrict__ out_em) {
-  extern __shared__ int32_t lds[];  // [max(local_n, 1)] histogram, [kAlignWaves][kAlignList] matches
-  align_workgroup<MAP, kAlignList>(topk_ids, expert_map, N, block_size, num_experts, local_n, max_EM,
-                                   sorted_ids, expert_ids, out_em, lds, lds + (local_n > 0 ? local_n : 1));
+  extern __shared__ int32_t lds[];  // [max(local_n, 1)] histogram, without ONE [kAlignWaves][kAlignList] matches
+  align_workgroup<MAP, ONE>(topk_ids, expert_map, N, block_size, num_experts, local_n, max_EM, sorted_ids,
+                            expert_ids, out_em, lds, lds + (local_n > 0 ? local_n : 1));
 }
 
 // Router and alignment in one launch, for decode-sized batches: every workgroup routes
@@ -250,8 +269,7 @@ __global__ __launch_bounds__(kAlignThreads) void route_align_kernel(
     int32_t* __restrict__ topk_ids, float* __restrict__ topk_w,
     int32_t* __restrict__ sorted_ids, int32_t* __restrict__ expert_ids,
     int32_t* __restrict__ out_em) {
-  // [max(local_n, 1)] histogram, [T * top_k] routing indices, [kAlignWaves][64] matches
-  extern __shared__ int32_t lds[];
+  extern __shared__ int32_t lds[];  // [max(local_n, 1)] histogram, [T * top_k] routing indices
   int32_t* const ids = lds + (local_n > 0 ? local_n : 1);
   const int lane = threadIdx.x & 63;
   for (int token = threadIdx.x >> 6; token < T; token += kAlignWaves) {  // uniform per wavefront
@@ -267,14 +285,12 @@ __global__ __launch_bounds__(kAlignThreads) void route_align_kernel(
     }
   }
   __syncthreads();
-  // (a wavefront's slice is one chunk of 64: T * top_k <= kRouteAlignMaxRows)
-  int32_t* const lists = ids + T * top_k;
   if (expert_map != nullptr)
-    align_workgroup<true, 64>(ids, expert_map, T * top_k, block_size, E, local_n, max_EM, sorted_ids,
-                              expert_ids, out_em, lds, lists);
+    align_workgroup<true, true>(ids, expert_map, T * top_k, block_size, E, local_n, max_EM, sorted_ids,
+                                expert_ids, out_em, lds, nullptr);
   else
-    align_workgroup<false, 64>(ids, nullptr, T * top_k, block_size, E, local_n, max_EM, sorted_ids, expert_ids,
-                               out_em, lds, lists);
+    align_workgroup<false, true>(ids, nullptr, T * top_k, block_size, E, local_n, max_EM, sorted_ids, expert_ids,
+                                 out_em, lds, nullptr);
 }
 
 }  // namespace
@@ -290,7 +306,7 @@ void launch_route_align(const float* logits, int T, int E, int top_k, int renorm
                         int32_t* topk_ids, float* topk_w, int32_t* sorted_ids, int32_t* expert_ids,
                         int32_t* out_em, hipStream_t stream) {
   const int groups = local_n > 0 ? local_n : 1;
-  const size_t lds = sizeof(int32_t) * ((size_t)groups + (size_t)T * (size_t)top_k + kAlignWaves * 64);
+  const size_t lds = sizeof(int32_t) * ((size_t)groups + (size_t)T * (size_t)top_k);
 #define VK_ROUTE_ALIGN_LAUNCH(PER)                                                                     \
   hipLaunchKernelGGL((route_align_kernel<PER>), dim3(groups), dim3(kAlignThreads), lds, stream, logits, \
                      T, E, top_k, renormalize, expert_map, block_size, local_n, max_EM, topk_ids,       \
@@ -309,13 +325,23 @@ void launch_align(const int32_t* topk_ids, const int32_t* expert_map, int N,
                   hipStream_t stream) {
   // local_n == 0 still needs one workgroup to write the sentinels and EM.
   const int groups = local_n > 0 ? local_n : 1;
-  const size_t lds = sizeof(int32_t) * ((size_t)groups + (size_t)kAlignList * kAlignWaves);
-  if (expert_map != nullptr)
-    hipLaunchKernelGGL(align_kernel<true>, dim3(groups), dim3(kAlignThreads), lds, stream, topk_ids, expert_map,
-                       N, block_size, num_experts, local_n, max_EM, sorted_ids, expert_ids, out_em);
-  else
-    hipLaunchKernelGGL(align_kernel<false>, dim3(groups), dim3(kAlignThreads), lds, stream, topk_ids, expert_map,
-                       N, block_size, num_experts, local_n, max_EM, sorted_ids, expert_ids, out_em);
+  // An index per lane up to kAlignThreads of them: a decode step's alignment is its launch, and
+  // walk and lists cost it 0.2 to 1 us (kernel times, walk -> lane: 4 indices 5.1 -> 4.6 us, 128
+  // 5.4 -> 5.0 us, 1024 with 128 experts 5.9 -> 5.0 us; in route_align_kernel 64 indices
+  // 7.6 -> 7.1 us).  1028 walk: 5.8 us.
+  const bool one = N <= kAlignThreads;
+  const size_t lds = sizeof(int32_t) * ((size_t)groups + (one ? 0 : (size_t)kAlignList * kAlignWaves));
+#define VK_ALIGN_LAUNCH(MAP, ONE)                                                                              \
+  hipLaunchKernelGGL((align_kernel<MAP, ONE>), dim3(groups), dim3(kAlignThreads), lds, stream, topk_ids,       \
+                     expert_map, N, block_size, num_experts, local_n, max_EM, sorted_ids, expert_ids, out_em)
+  if (expert_map != nullptr) {
+    if (one) VK_ALIGN_LAUNCH(true, true);
+    else VK_ALIGN_LAUNCH(true, false);
+  } else {
+    if (one) VK_ALIGN_LAUNCH(false, true);
+    else VK_ALIGN_LAUNCH(false, false);
+  }
+#undef VK_ALIGN_LAUNCH
 }
 
 }  // namespace vk
