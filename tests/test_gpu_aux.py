@@ -121,6 +121,54 @@ def test_scatter_reduce_on_a_used_workspace(hip_lib, top_k):
         assert np.array_equal(out.cpu().numpy().view(np.uint32), ref.view(np.uint32))
 
 
+@pytest.mark.parametrize("top_k", [1, 2, 3, 4, 5, 6, 7, 8, 9, 16])
+def test_all_combines_on_a_used_workspace(hip_lib, top_k):
+    """scatter_reduce, scatter_reduce_q and moe_combine (bias, a block without an expert) for every
+    number of experts per token they are compiled for and for others, on workspaces that hold what
+    an earlier call left there."""
+    sr, srq, mc = (getattr(hip_lib, n) for n in ("vk_hip_mxfp4_moe_scatter_reduce",
+                                                 "vk_hip_mxfp4_moe_scatter_reduce_q", "vk_hip_moe_combine"))
+    sr.restype = srq.restype = mc.restype = _I
+    sr.argtypes = [_P] * 4 + [_I] * 4 + [_P, ctypes.c_size_t, _P]
+    srq.argtypes = [_P] * 5 + [_I] * 5 + [_P, ctypes.c_size_t, _P]
+    mc.argtypes = [_P] * 6 + [_I] * 5 + [_P, ctypes.c_size_t, _P]
+    rng = np.random.default_rng(100 + top_k)
+    M, E, width = 53, 16, 192          # (the oracle's moe_combine takes whole tiles of 64 columns)
+    ids = np.stack([rng.permutation(E)[:top_k] for _ in range(M)]).astype(np.int32)
+    emap = np.where(np.arange(E) % 4 == 1, -1, np.cumsum(np.arange(E) % 4 != 1) - 1).astype(np.int32)
+    sids, eids, em = oracle.moe_align_block_size_with_map(ids.ravel(), E, 16, emap)
+    sids, eids = sids[:em].copy(), eids[:em // 16].copy()
+    eids[len(eids) // 2] = -1
+    partial = rng.standard_normal((em, width)).astype(np.float32)
+    bias = rng.standard_normal((E, width)).astype(np.float32)
+    fin = np.array(synth.FINITE_CODES, np.uint8)
+    pq = fin[rng.integers(0, 12, (em, width // 2))] | (fin[rng.integers(0, 12, (em, width // 2))] << 4)
+    ps = rng.integers(110, 140, (em, width // 32)).astype(np.uint8)
+    ps[rng.random(ps.shape) < 0.1] = 0xFF
+    tws = rng.random(em).astype(np.float32)
+    base = rng.standard_normal((M, width)).astype(np.float32)
+    refs = (oracle.mxfp4_moe_scatter_reduce(partial, tws, sids, M, top_k, out=base.copy()),
+            oracle.mxfp4_moe_scatter_reduce_q(pq, ps, tws, sids, M, top_k, out=base.copy()),
+            oracle.moe_combine(partial, bias, tws, sids, eids, M, width, top_k, em, out=base.copy()))
+    d_p, d_b, d_pq, d_ps, d_w, d_s, d_e = (to_dev(a) for a in (partial, bias, pq, ps, tws, sids, eids))
+    for garbage in (np.arange(M * top_k) % em, np.full(M * top_k, em),
+                    np.repeat(np.arange(M) % em, top_k), rng.integers(-2 ** 31, 2 ** 31, M * top_k)):
+        for i, ref in enumerate(refs):
+            ws, out = to_dev(garbage.astype(np.int32)), to_dev(base.copy())
+            scratch = (ws.data_ptr(), ws.numel() * 4, None)
+            if i == 0:
+                rc = sr(d_p.data_ptr(), d_w.data_ptr(), d_s.data_ptr(), out.data_ptr(), M, width, top_k, em, *scratch)
+            elif i == 1:
+                rc = srq(d_pq.data_ptr(), d_ps.data_ptr(), d_w.data_ptr(), d_s.data_ptr(), out.data_ptr(), M, width,
+                         top_k, em, 32, *scratch)
+            else:
+                rc = mc(d_p.data_ptr(), d_b.data_ptr(), d_w.data_ptr(), d_s.data_ptr(), d_e.data_ptr(),
+                        out.data_ptr(), M, width, top_k, em, 16, *scratch)
+            assert rc == 0
+            torch.cuda.synchronize()
+            assert np.array_equal(out.cpu().numpy().view(np.uint32), ref.view(np.uint32)), i
+
+
 def test_sorted_quant_and_scatter_reduce_bitwise(hip_lib):
     sq = hip_lib.vk_hip_mxfp4_moe_sorted_quant
     sq.restype = _I

@@ -48,10 +48,9 @@ __global__ __launch_bounds__(256) void act_epilogue_kernel(
 }
 
 // pos[flat] = sorted row of every routed flat index.  The entries of the others hold
-// whatever the caller's workspace held: the combines take an entry only when sorted_ids says
-// that its row is that flat index's (routed_row), which saves the launch that would clear the
-// table (4.7 us and the gap before it, of 215 us for the orchestration ops around 4096 tokens
-// of 4096 and of 298 us for a tensor-parallel rank's share of 2048).
+// whatever the caller's workspace held: the combines for a known number of experts per token
+// take an entry only when sorted_ids says that its row is that flat index's (routed_row),
+// which saves the launch that would clear the table (4.7 us and the gap before it).
 __global__ __launch_bounds__(256) void invert_sorted_ids_kernel(const int32_t* __restrict__ sorted_ids,
                                                                 int32_t* __restrict__ pos, int EM,
                                                                 int n_flat) {
@@ -90,14 +89,43 @@ __device__ __forceinline__ void sorted_rows(const int32_t* __restrict__ pos,
   for (int j = 0; j < TOPK; ++j) rows[j] = (int)key[j];
 }
 
+// The combines for any number of experts per token: use(r) over the token's sorted rows in
+// ascending order, the next one looked for among the entries of a cleared table (an entry is
+// asked for top_k times, so a check of each against sorted_ids costs more than the launch that
+// clears: 4096 tokens x 10 rows of 4096, 152 us with both and 243 us with checked entries).
+template <class Use>
+__device__ __forceinline__ void for_each_row(const int32_t* __restrict__ pos, int t, int top_k, Use&& use) {
+  int last = -1;
+  for (int s = 0; s < top_k; ++s) {
+    int r = 0x7FFFFFFF;
+    for (int j = 0; j < top_k; ++j) {
+      const int rj = pos[t * top_k + j];
+      if (rj > last && rj < r) r = rj;
+    }
+    if (r == 0x7FFFFFFF) break;
+    last = r;
+    use(r);
+  }
+}
+
+// Numbers of experts per token that the combines are compiled for; others clear the table.
+// Rows found once and asked for together, against the search over a cleared table (launches of
+// one call of 4096 tokens, rows of 4096, in all): 7 rows 127 -> 104 us, 8 rows 138 -> 117 us;
+// quantised rows 4 a token 49 -> 42 us, 8 a token 90 -> 70 us.
+#define VK_COMBINE_TOPK(X) X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(8)
+
 // Routed combine in gather form: out[t, :] += (partial[r, :] + bias[e(r), :]) * w[r] over
 // the token's sorted rows r in ascending order, which is the order the reference's loops
 // over the rows add them in (moe_combine_cpu, moe_fused.cpp:523-564; without a bias,
 // mxfp4_moe_scatter_reduce, moe_aux.cpp:265-285).  The sum with the bias, the product and
 // the sum into out are each rounded on their own, as there, so the result is the
 // reference's bit for bit.  A row of a block without an expert (expert_ids given) adds
-// nothing.  One thread per 4 columns.
-template <int TOPK>  // experts per token, 0 = any number (the next row looked for one at a time)
+// nothing.  One thread per 4 columns.  The rows are read once, past the caches: 4096 tokens of
+// 4096 columns 3 us faster for 4 rows a token and 20 us for 8; behind the linear stages of a
+// rank of four the call in all 123.5 -> 122.8 us for 512 tokens x 6, 527 -> 508 us for 4096 x 6.
+// Rows that a caller's GEMM has just left in the last cache are read 3 us slower (4096 x 1:
+// 28.5 -> 31.4 us).
+template <int TOPK>  // experts per token, 0 = any number (for_each_row)
 __global__ __launch_bounds__(256) void combine_rows_kernel(
     const float* __restrict__ partial, const float* __restrict__ bias, const float* __restrict__ w_sorted,
     const int32_t* __restrict__ pos, const int32_t* __restrict__ sorted_ids,
@@ -134,17 +162,7 @@ __global__ __launch_bounds__(256) void combine_rows_kernel(
       for (int s = 0; s < TOPK; ++s)
         if (rows[s] >= 0) add(p[s], rows[s]);
     } else {
-      int last = -1;
-      for (int s = 0; s < top_k; ++s) {   // the next larger sorted row of this token (top_k is small)
-        int r = 0x7FFFFFFF;
-        for (int j = 0; j < top_k; ++j) {
-          const int rj = routed_row(pos, sorted_ids, t * top_k + j, EM);
-          if (rj > last && rj < r) r = rj;
-        }
-        if (r == 0x7FFFFFFF) break;
-        last = r;
-        add(load(r), r);
-      }
+      for_each_row(pos, t, top_k, [&](int r) { add(load(r), r); });
     }
     *o = sum;
   }
@@ -181,6 +199,7 @@ __global__ __launch_bounds__(256) void gather_rows_kernel(const uint8_t* __restr
 // (moe_aux.cpp:76-82: the bits s << 23).  The dequantised value, its product with the
 // routing weight and the sum into out are each rounded on their own, as there.  Gather
 // form over the table of sorted positions; one thread per 8 columns (4 bytes of codes).
+template <int TOPK>
 __global__ __launch_bounds__(256) void combine_rows_q_kernel(
     const uint8_t* __restrict__ partial_q, const uint8_t* __restrict__ partial_s,
     const float* __restrict__ w_sorted, const int32_t* __restrict__ pos,
@@ -193,17 +212,11 @@ __global__ __launch_bounds__(256) void combine_rows_q_kernel(
     float sum[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) sum[i] = o[i];
-    int last = -1;
-    for (int s = 0; s < top_k; ++s) {   // the next larger sorted row of this token (top_k is small)
-      int r = 0x7FFFFFFF;
-      for (int j = 0; j < top_k; ++j) {
-        const int rj = routed_row(pos, sorted_ids, t * top_k + j, EM);
-        if (rj > last && rj < r) r = rj;
-      }
-      if (r == 0x7FFFFFFF) break;
-      last = r;
-      const uint32_t codes = *reinterpret_cast<const uint32_t*>(partial_q + (size_t)r * (size_t)(width / 2) + c / 2);
-      const uint32_t sb = partial_s[(size_t)r * (size_t)groups + c / 32];
+    auto load = [&](int r, uint32_t& codes, uint32_t& sb) {
+      codes = *reinterpret_cast<const uint32_t*>(partial_q + (size_t)r * (size_t)(width / 2) + c / 2);
+      sb = partial_s[(size_t)r * (size_t)groups + c / 32];
+    };
+    auto add = [&](uint32_t codes, uint32_t sb, int r) {
       const float scale = sb == 0xFFu ? 0.0f : __uint_as_float(sb << 23);
       const float w = w_sorted[r];
 #pragma unroll
@@ -214,10 +227,41 @@ __global__ __launch_bounds__(256) void combine_rows_q_kernel(
         asm volatile("" : "+v"(prod));
         sum[i] += prod;
       }
+    };
+    if constexpr (TOPK > 0) {
+      int rows[TOPK];
+      sorted_rows<TOPK>(pos, sorted_ids, t, EM, rows);
+      uint32_t codes[TOPK], sb[TOPK];
+#pragma unroll
+      for (int s = 0; s < TOPK; ++s) load(rows[s] < 0 ? 0 : rows[s], codes[s], sb[s]);
+#pragma unroll
+      for (int s = 0; s < TOPK; ++s)
+        if (rows[s] >= 0) add(codes[s], sb[s], rows[s]);
+    } else {
+      for_each_row(pos, t, top_k, [&](int r) {
+        uint32_t codes, sb;
+        load(r, codes, sb);
+        add(codes, sb, r);
+      });
     }
 #pragma unroll
     for (int i = 0; i < 8; ++i) o[i] = sum[i];
   }
+}
+
+// The table of sorted positions for a combine over top_k experts per token.
+void launch_invert_sorted_ids(const int32_t* sorted_ids, int32_t* pos, int EM, int M, int top_k,
+                              hipStream_t stream) {
+  switch (top_k) {
+#define VK_KNOWN(K_) case K_:
+    VK_COMBINE_TOPK(VK_KNOWN)
+#undef VK_KNOWN
+      break;
+    default:
+      launch_fill_i32(pos, -1, M * top_k, stream);
+  }
+  hipLaunchKernelGGL(invert_sorted_ids_kernel, dim3((unsigned)((EM + 255) / 256)), dim3(256), 0, stream,
+                     sorted_ids, pos, EM, M * top_k);
 }
 
 }  // namespace
@@ -241,11 +285,20 @@ void launch_mxfp4_scatter_reduce_q(const uint8_t* partial_q, const uint8_t* part
                                    const int32_t* sorted_ids, float* out, int M, int width, int top_k,
                                    int EM, int32_t* pos, hipStream_t stream) {
   if (M <= 0 || width <= 0 || EM <= 0) return;
-  hipLaunchKernelGGL(invert_sorted_ids_kernel, dim3((unsigned)((EM + 255) / 256)), dim3(256), 0, stream,
-                     sorted_ids, pos, EM, M * top_k);
+  launch_invert_sorted_ids(sorted_ids, pos, EM, M, top_k, stream);
   const dim3 grid((unsigned)((width / 8 + 255) / 256), (unsigned)(M < 65535 ? M : 65535));
-  hipLaunchKernelGGL(combine_rows_q_kernel, grid, dim3(256), 0, stream, partial_q, partial_s, topk_w, pos,
-                     sorted_ids, out, M, width, top_k, EM);
+  switch (top_k) {
+#define VK_COMBINE(K_)                                                                                  \
+  case K_:                                                                                              \
+    hipLaunchKernelGGL(combine_rows_q_kernel<K_>, grid, dim3(256), 0, stream, partial_q, partial_s,     \
+                       topk_w, pos, sorted_ids, out, M, width, top_k, EM);                              \
+    break;
+    VK_COMBINE_TOPK(VK_COMBINE)
+#undef VK_COMBINE
+    default:
+      hipLaunchKernelGGL(combine_rows_q_kernel<0>, grid, dim3(256), 0, stream, partial_q, partial_s, topk_w,
+                         pos, sorted_ids, out, M, width, top_k, EM);
+  }
 }
 
 void launch_moe_act_epilogue(const float* gate_up, const float* b13, uint16_t* act,
@@ -264,8 +317,7 @@ void launch_moe_combine_sorted(const float* partial, const float* bias, const fl
                                int width, int top_k, int EM, int block_size, int32_t* pos,
                                hipStream_t stream) {
   if (M <= 0 || width <= 0 || EM <= 0) return;
-  hipLaunchKernelGGL(invert_sorted_ids_kernel, dim3((unsigned)((EM + 255) / 256)), dim3(256), 0, stream,
-                     sorted_ids, pos, EM, M * top_k);
+  launch_invert_sorted_ids(sorted_ids, pos, EM, M, top_k, stream);
   const dim3 grid((unsigned)((width / 4 + 255) / 256), (unsigned)(M < 65535 ? M : 65535));
   const int bs = block_size > 0 ? block_size : 16;
   switch (top_k) {
@@ -274,7 +326,7 @@ void launch_moe_combine_sorted(const float* partial, const float* bias, const fl
     hipLaunchKernelGGL(combine_rows_kernel<K_>, grid, dim3(256), 0, stream, partial, bias, w_sorted, pos, \
                        sorted_ids, expert_ids, out, M, width, top_k, EM, bs);                            \
     break;
-    VK_COMBINE(1) VK_COMBINE(2) VK_COMBINE(4) VK_COMBINE(6) VK_COMBINE(8)
+    VK_COMBINE_TOPK(VK_COMBINE)
 #undef VK_COMBINE
     default:
       hipLaunchKernelGGL(combine_rows_kernel<0>, grid, dim3(256), 0, stream, partial, bias, w_sorted, pos,
