@@ -93,6 +93,42 @@ def test_quant_widths_and_magnitudes_bitwise(hip_lib, hidden):
     assert np.array_equal(scales.cpu().numpy(), rs) and np.array_equal(packed.cpu().numpy(), rp)
 
 
+@pytest.mark.parametrize("hidden,rows", [(2048, 3), (2080, 1), (2080, 4096), (2080, 4097), (4096, 65),
+                                         (7168, 17), (8224, 2)])
+def test_quant_a_workgroup_per_row_at_its_edges(hip_lib, hidden, rows):
+    """Rows of one piece more than a wavefront takes in a batch, the most rows that have a
+    workgroup each and one more, in token order and in sorted order with padding between."""
+    q, sq = hip_lib.vk_hip_mxfp4_moe_quant, hip_lib.vk_hip_mxfp4_moe_sorted_quant
+    q.restype = sq.restype = _I
+    q.argtypes = [_P] * 3 + [_I] * 3 + [_P]
+    sq.argtypes = [_P] * 4 + [_I] * 5 + [_P]
+    rng = np.random.default_rng(hidden + rows)
+    A = synth.f32_to_bf16_bits((rng.standard_normal((rows, hidden)) * 2.0 ** rng.integers(-120, 100, (rows, 1)))
+                               .astype(np.float32))
+    A[rng.integers(0, rows, 9), rng.integers(0, hidden, 9)] = 0x7FC0     # NaN, infinities, zero groups
+    A[rng.integers(0, rows, 9), rng.integers(0, hidden, 9)] = 0xFF80
+    A[rows - 1, hidden - 32:] = 0x8000
+    packed = torch.full((rows + 1, hidden // 2), 7, dtype=torch.uint8, device=dev())
+    scales = torch.full((rows + 1, hidden // 32), 7, dtype=torch.uint8, device=dev())
+    d_A = to_dev(A)
+    assert q(d_A.data_ptr(), packed.data_ptr(), scales.data_ptr(), rows, hidden, 32, None) == 0
+    torch.cuda.synchronize()
+    rp, rs = oracle.mxfp4_moe_quant(A)
+    assert np.array_equal(packed.cpu().numpy(), np.r_[rp, np.full((1, hidden // 2), 7, np.uint8)])
+    assert np.array_equal(scales.cpu().numpy(), np.r_[rs, np.full((1, hidden // 32), 7, np.uint8)])
+    sids = rng.integers(0, 2 * rows, rows).astype(np.int32)              # top_k 1: half of them padding
+    sids[rng.random(rows) < 0.1] = -5
+    packed.fill_(7)
+    scales.fill_(7)
+    d_s = to_dev(sids)
+    assert sq(d_A.data_ptr(), d_s.data_ptr(), packed.data_ptr(), scales.data_ptr(), rows, hidden, 32, 1, rows,
+              None) == 0
+    torch.cuda.synchronize()
+    rp, rs = oracle.mxfp4_moe_sorted_quant(A, sids, 1)
+    assert np.array_equal(packed.cpu().numpy(), np.r_[rp, np.full((1, hidden // 2), 7, np.uint8)])
+    assert np.array_equal(scales.cpu().numpy(), np.r_[rs, np.full((1, hidden // 32), 7, np.uint8)])
+
+
 @pytest.mark.parametrize("top_k", [1, 2, 3, 4, 6, 8])
 def test_scatter_reduce_on_a_used_workspace(hip_lib, top_k):
     """The table of sorted positions holds what an earlier call left there: flat indices without

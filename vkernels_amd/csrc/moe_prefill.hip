@@ -418,19 +418,19 @@ __device__ __forceinline__ void quant_quad_any(const u32x4& v, uint32_t& sb, uin
 // store(i, codes, scale byte).  A few loads are issued together (one at a time is a round
 // trip to memory for every 8 values); the groups the packed routine does not take are done
 // over afterwards, where they occur, so that their code stands here once and out of the way.
+constexpr int kQuantBatch = 4;
 template <typename Load, typename Store>
 __device__ __forceinline__ void quant_row(int first, int step, int pieces, Load load, Store store) {
-  constexpr int kBatch = 4;
-  for (int i0 = first; i0 < pieces; i0 += kBatch * step) {
-    u32x4 v[kBatch];
+  for (int i0 = first; i0 < pieces; i0 += kQuantBatch * step) {
+    u32x4 v[kQuantBatch];
 #pragma unroll
-    for (int j = 0; j < kBatch; ++j) {
+    for (int j = 0; j < kQuantBatch; ++j) {
       v[j] = u32x4{0u, 0u, 0u, 0u};
       if (i0 + j * step < pieces) v[j] = load(i0 + j * step);
     }
     bool all = true;
 #pragma unroll
-    for (int j = 0; j < kBatch; ++j) {
+    for (int j = 0; j < kQuantBatch; ++j) {
       if (i0 + j * step >= pieces) break;
       uint32_t sb, codes;
       if (quant_quad(v[j], sb, codes)) store(i0 + j * step, codes, sb);
@@ -438,7 +438,7 @@ __device__ __forceinline__ void quant_row(int first, int step, int pieces, Load 
     }
     if (all) continue;
 #pragma unroll 1
-    for (int i = i0; i < min(i0 + kBatch * step, pieces); i += step) {
+    for (int i = i0; i < min(i0 + kQuantBatch * step, pieces); i += step) {
       const u32x4 w = load(i);
       uint32_t sb, codes;
       quant_quad_any(w, sb, codes);  // (any group: the same codes where the packed routine has been)
@@ -454,24 +454,47 @@ __host__ __device__ constexpr int quant_lane_bits(int pieces) {
   while (bits < 6 && (1 << bits) < pieces) ++bits;
   return bits;
 }
-static inline dim3 quant_grid(int rows, int pieces) {
-  const int per_group = 4 * (64 >> quant_lane_bits(pieces));  // 4 wavefronts
+// A row that is more than one batch for each of a wavefront's lanes takes a workgroup (WIDE)
+// while rows are few: a wavefront goes through its batches one after the other, and few rows
+// leave the rest of the device idle meanwhile.  Kernel times, a wavefront -> a workgroup a row:
+// width 7168, 1 row 5.1 -> 2.2 us, 256 rows 6.5 -> 3.3 us, 4032 sorted rows 14.3 -> 12.2 us;
+// 2880, 64 rows 4.0 -> 2.6 us, 4032 sorted rows 7.8 -> 7.3 us; beyond 4096 rows from 4 % ahead
+// (25536 of 4096) to 10 % behind (25536 of 2880).  Rows of one batch or less were 0.4 to 1 us
+// ahead up to a thousand and up to 45 % behind beyond.
+constexpr int kQuantWidePieces = 64 * kQuantBatch, kQuantWideRows = 4096;
+static inline bool quant_wide(int rows, int pieces) { return rows <= kQuantWideRows && pieces > kQuantWidePieces; }
+static inline dim3 quant_grid(int rows, int pieces, bool wide) {
+  const int per_group = wide ? 1 : 4 * (64 >> quant_lane_bits(pieces));  // 4 wavefronts
   return dim3((unsigned)((rows + per_group - 1) / per_group));
+}
+// The row of this lane and the first of its pieces and their step.
+template <bool WIDE>
+__device__ __forceinline__ size_t quant_row_of_lane(int pieces, int& first, int& step) {
+  if constexpr (WIDE) {
+    first = threadIdx.x;
+    step = 256;
+    return blockIdx.x;
+  }
+  const int bits = quant_lane_bits(pieces);
+  const int lane = threadIdx.x & 63;
+  step = 1 << bits;
+  first = lane & (step - 1);
+  return (size_t)(blockIdx.x * 4 + (threadIdx.x >> 6)) * (size_t)(64 >> bits) + (size_t)(lane >> bits);
 }
 
 // Packed codes [rows, K/2] and scale bytes [rows, K/32] of bf16 rows: row r of the output
 // is x[r] (sorted_ids null) or x[sorted_ids[r] / top_k], a padding row (id outside
 // [0, n_flat)) giving zero codes and 0xFF scales (mxfp4_moe_sorted_quant,
 // moe_aux.cpp:171-209).
+template <bool WIDE>
 __global__ __launch_bounds__(256) void mxfp4_quant_kernel(const uint16_t* __restrict__ x,
                                                           const int32_t* __restrict__ sorted_ids,
                                                           uint8_t* __restrict__ packed,
                                                           uint8_t* __restrict__ scales, int K, int rows,
                                                           int top_k, int n_flat) {
   const int pieces = K / 8;
-  const int bits = quant_lane_bits(pieces);
-  const int lane = threadIdx.x & 63;
-  const size_t row = (size_t)(blockIdx.x * 4 + (threadIdx.x >> 6)) * (size_t)(64 >> bits) + (size_t)(lane >> bits);
+  int first, step;
+  const size_t row = quant_row_of_lane<WIDE>(pieces, first, step);
   if (row >= (size_t)rows) return;
   const uint16_t* src = x + row * (size_t)K;
   bool pad = false;
@@ -482,7 +505,6 @@ __global__ __launch_bounds__(256) void mxfp4_quant_kernel(const uint16_t* __rest
   }
   uint8_t* const prow = packed + row * (size_t)(K / 2);
   uint8_t* const srow = scales + row * (size_t)(K / 32);
-  const int step = 1 << bits, first = lane & (step - 1);
   auto store = [&](int i, uint32_t codes, uint32_t sb) {
     *reinterpret_cast<uint32_t*>(prow + (size_t)i * 4) = codes;
     if ((i & 3) == 0) srow[i >> 2] = (uint8_t)sb;
@@ -500,6 +522,7 @@ __global__ __launch_bounds__(256) void mxfp4_quant_kernel(const uint16_t* __rest
 // byte is outside the range the scaled MFMA path takes.  8191 tokens x 6 rows of 1536:
 // 169 -> 59 us (4.1 TB/s) with as many rows a wavefront as it has lanes for (a workgroup per row left
 // four fifths of it idle) and the packed quantisation.
+template <bool WIDE>
 __global__ __launch_bounds__(256) void quant_rows_w4_kernel(const uint16_t* __restrict__ x,
                                                             uint8_t* __restrict__ xq,
                                                             uint8_t* __restrict__ row_bad, int K, int rows,
@@ -509,9 +532,8 @@ __global__ __launch_bounds__(256) void quant_rows_w4_kernel(const uint16_t* __re
   for (int i = (int)(blockIdx.x * 256 + threadIdx.x); i < fill_n; i += (int)(gridDim.x * 256)) fill[i] = -1;
   const int kp = mx_kp(K);
   const int pieces = kp / 8;
-  const int bits = quant_lane_bits(pieces);
-  const int lane = threadIdx.x & 63;
-  const size_t row = (size_t)(blockIdx.x * 4 + (threadIdx.x >> 6)) * (size_t)(64 >> bits) + (size_t)(lane >> bits);
+  int first, step;
+  const size_t row = quant_row_of_lane<WIDE>(pieces, first, step);
   if (row >= (size_t)rows) return;
   if (sorted_ids != nullptr) {  // as split_rows_fp6_kernel: routed rows only
     const int f = sorted_ids[row];
@@ -519,7 +541,6 @@ __global__ __launch_bounds__(256) void quant_rows_w4_kernel(const uint16_t* __re
   }
   uint8_t* qrow = xq + row * (size_t)kp;
   const uint16_t* src = x + row * (size_t)K;
-  const int step = 1 << bits, first = lane & (step - 1);
   bool bad = false;
   auto load = [&](int i) {
     u32x4 v = {0u, 0u, 0u, 0u};
@@ -540,10 +561,15 @@ __global__ __launch_bounds__(256) void quant_rows_w4_kernel(const uint16_t* __re
     *reinterpret_cast<u32x2*>(qrow + (size_t)(i >> 2) * 32 + (i & 3) * 8) = u32x2{w0, w1};
   };
   quant_row(first, step, pieces, load, store);
-  // the row's lanes are `step` consecutive ones (all of them here, or none: a row's lanes leave together)
-  const unsigned long long any = __ballot(bad);
-  const unsigned long long mine = (step == 64 ? ~0ull : ((1ull << step) - 1ull) << (lane & ~(step - 1)));
-  if (first == 0) row_bad[row] = (uint8_t)((any & mine) != 0ull);
+  if constexpr (WIDE) {
+    bad = __syncthreads_or(bad);  // (the workgroup's row is one: all its lanes are here, or none)
+    if (first == 0) row_bad[row] = (uint8_t)bad;
+  } else {
+    // the row's lanes are `step` consecutive ones (all of them here, or none: a row's lanes leave together)
+    const unsigned long long any = __ballot(bad);
+    const unsigned long long mine = (step == 64 ? ~0ull : ((1ull << step) - 1ull) << (threadIdx.x & 63 & ~(step - 1)));
+    if (first == 0) row_bad[row] = (uint8_t)((any & mine) != 0ull);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1318,9 +1344,21 @@ bool mx_plan(const FusedMoeArgs& a, bool need_stage0, MxPlan& pl) {
   return true;
 }
 
+void launch_quant_rows_w4(const uint16_t* x, uint8_t* xq, uint8_t* row_bad, int K, int rows,
+                          const int32_t* sorted_ids, int n_flat, int32_t* fill, int fill_n, hipStream_t stream) {
+  const int pieces = mx_kp(K) / 8;
+  // (the rows of the sorted order that are not routed leave at once: they do not count)
+  if (quant_wide(sorted_ids != nullptr && n_flat < rows ? n_flat : rows, pieces))
+    hipLaunchKernelGGL(quant_rows_w4_kernel<true>, quant_grid(rows, pieces, true), dim3(256), 0, stream, x, xq,
+                       row_bad, K, rows, sorted_ids, n_flat, fill, fill_n);
+  else
+    hipLaunchKernelGGL(quant_rows_w4_kernel<false>, quant_grid(rows, pieces, false), dim3(256), 0, stream, x, xq,
+                       row_bad, K, rows, sorted_ids, n_flat, fill, fill_n);
+}
+
 void mx_stage0(const FusedMoeArgs& a, const MxPlan& pl, hipStream_t stream) {
   if (pl.terms0 == 1) {
-    hipLaunchKernelGGL(quant_rows_w4_kernel, quant_grid(a.M, mx_kp(a.hidden) / 8), dim3(256), 0, stream, a.A, pl.aq, pl.abad, a.hidden, a.M, nullptr, 0, nullptr, 0);
+    launch_quant_rows_w4(a.A, pl.aq, pl.abad, a.hidden, a.M, nullptr, 0, nullptr, 0, stream);
     launch_mx_stage_t<0, 1>(pl.g0, stream);
   } else if (pl.terms0 == 2) {
     hipLaunchKernelGGL(split_rows_fp6_kernel<2>, split_grid(a.M, a.hidden), dim3(256), 0, stream, a.A, pl.aq, pl.abad, a.hidden, a.hidden, a.M, nullptr, 0, nullptr, 0);
@@ -1335,7 +1373,8 @@ void mx_stage0(const FusedMoeArgs& a, const MxPlan& pl, hipStream_t stream) {
 // sorted positions) -> second stage -> per-token sum
 void mx_stage1(const FusedMoeArgs& a, const MxPlan& pl, hipStream_t stream) {
   if (pl.terms1 == 1) {
-    hipLaunchKernelGGL(quant_rows_w4_kernel, quant_grid(a.EM, mx_kp(a.ispp) / 8), dim3(256), 0, stream, a.act, pl.cq, pl.cbad, a.ispp, a.EM, a.sorted_ids, a.M * a.top_k, pl.pos, a.M * a.top_k);
+    launch_quant_rows_w4(a.act, pl.cq, pl.cbad, a.ispp, a.EM, a.sorted_ids, a.M * a.top_k, pl.pos, a.M * a.top_k,
+                         stream);
     launch_mx_stage_t<1, 1>(pl.g1, stream);
   } else if (pl.terms1 == 2) {
     hipLaunchKernelGGL(split_rows_fp6_kernel<2>, split_grid(a.EM, a.ispp), dim3(256), 0, stream, a.act, pl.cq, pl.cbad, a.ispp, a.ispp, a.EM, a.sorted_ids, a.M * a.top_k, pl.pos, a.M * a.top_k);
@@ -1458,8 +1497,13 @@ void launch_split_rows_fp6(const uint16_t* x, int rows, int K, int terms, uint8_
 void launch_mxfp4_quant(const uint16_t* A, const int32_t* sorted_ids, uint8_t* packed, uint8_t* scales,
                         int rows, int hidden, int top_k, int n_flat, hipStream_t stream) {
   if (rows <= 0 || hidden <= 0) return;
-  hipLaunchKernelGGL(mxfp4_quant_kernel, quant_grid(rows, hidden / 8), dim3(256), 0, stream, A, sorted_ids,
-                     packed, scales, hidden, rows, top_k, n_flat);
+  const int pieces = hidden / 8;
+  if (quant_wide(rows, pieces))
+    hipLaunchKernelGGL(mxfp4_quant_kernel<true>, quant_grid(rows, pieces, true), dim3(256), 0, stream, A, sorted_ids,
+                       packed, scales, hidden, rows, top_k, n_flat);
+  else
+    hipLaunchKernelGGL(mxfp4_quant_kernel<false>, quant_grid(rows, pieces, false), dim3(256), 0, stream, A,
+                       sorted_ids, packed, scales, hidden, rows, top_k, n_flat);
 }
 
 }  // namespace vk
