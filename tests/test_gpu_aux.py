@@ -17,7 +17,8 @@ from vkernels_amd import synth
 from vkernels_amd import vllm_experts as ve
 
 import test_gpu_configs as cfgs
-from gpu_util import MAX_ABS_TOL, REL_L2_TOL, cpu_layer, dev, edge_tokens, error_metrics, to_dev
+from gpu_util import (EXACT_SPLIT_MAX_ABS_TOL, EXACT_SPLIT_REL_L2_TOL, MAX_ABS_TOL, REL_L2_TOL, cpu_layer, dev,
+                      edge_tokens, error_metrics, to_dev)
 
 pytestmark = pytest.mark.gpu
 
@@ -203,6 +204,30 @@ def test_all_combines_on_a_used_workspace(hip_lib, top_k):
             assert rc == 0
             torch.cuda.synchronize()
             assert np.array_equal(out.cpu().numpy().view(np.uint32), ref.view(np.uint32)), i
+
+
+@pytest.mark.parametrize("hidden", [32, 64, 96, 160, 256])
+def test_sorted_quant_of_rows_that_share_a_wavefront(hip_lib, hidden):
+    """2 to 16 rows to a wavefront: routed rows, padding and negative ids side by side, the last
+    workgroup not full, groups that only the general routine takes beside others."""
+    sq = hip_lib.vk_hip_mxfp4_moe_sorted_quant
+    sq.restype = _I
+    sq.argtypes = [_P, _P, _P, _P, _I, _I, _I, _I, _I, _P]
+    rng = np.random.default_rng(hidden)
+    M, top_k, em = 70, 3, 16 * 19 + 5
+    A = _edge_rows(M, 64, 303)[:, :32] if hidden == 32 else _edge_rows(M, hidden, 303)
+    sids = rng.integers(0, M * top_k, em).astype(np.int32)
+    sids[rng.random(em) < 0.4] = M * top_k
+    sids[rng.random(em) < 0.1] = -1
+    packed = torch.full((em + 1, hidden // 2), 7, dtype=torch.uint8, device=dev())
+    scales = torch.full((em + 1, hidden // 32), 7, dtype=torch.uint8, device=dev())
+    d_A, d_s = to_dev(A), to_dev(sids)
+    assert sq(d_A.data_ptr(), d_s.data_ptr(), packed.data_ptr(), scales.data_ptr(), M, hidden, 32, top_k, em,
+              None) == 0
+    torch.cuda.synchronize()
+    rp, rs = oracle.mxfp4_moe_sorted_quant(A, sids, top_k)
+    assert np.array_equal(packed.cpu().numpy(), np.r_[rp, np.full((1, hidden // 2), 7, np.uint8)])
+    assert np.array_equal(scales.cpu().numpy(), np.r_[rs, np.full((1, hidden // 32), 7, np.uint8)])
 
 
 def test_sorted_quant_and_scatter_reduce_bitwise(hip_lib):
@@ -399,3 +424,54 @@ def test_w4a4_rows_outside_the_range_take_the_exact_path():
     for t in range(T):
         max_rel, rel_l2, nf = error_metrics(g["out"][t], c["out"][t])
         assert nf and max_rel <= MAX_ABS_TOL and rel_l2 <= REL_L2_TOL, (t, max_rel, rel_l2)
+
+
+@pytest.mark.parametrize("H,I", [(256, 64), (320, 128), (192, 192), (2304, 2176)])
+def test_w4a4_stages_at_narrow_widths(H, I):
+    """Second-stage rows that share a wavefront or have a workgroup each, widths that are no
+    multiple of 128, and rows outside the range of the scaled products (their flag is per row)
+    beside rows inside it, in the first stage, in the second or in both.  Each stage against the
+    oracle on the same quantised operands, the second on the device's own act: the order of the
+    fp32 sums is all that differs, and the bf16 rounding of act in the first stage."""
+    cfg = synth.MoEConfig("t", H, I, 8, 2, (300,), "uniform")
+    T, seed = 300, 6400 + I
+    n_flat = T * cfg.top_k
+    w = synth.make_weights(cfg.E, H, I, seed, device=dev())
+    A, lg = cfgs._inputs(cfg, T, seed)
+    # scale bytes beyond 64 .. 190: A's at 2^-66, act's at 2^-66, 2^-40 and 2^35
+    power = np.array([0, 35, 0, -40, 0, -66, 20])[np.arange(T) % 7]
+    A = synth.f32_to_bf16_bits((synth.bf16_bits_to_f32(A) * np.exp2(power)[:, None]).astype(np.float32))
+    g = cfgs._run_gpu(cfg, w, A, lg, None, True, prepack=True, w4a4=True)
+    ids, tw = oracle.route_topk(lg, cfg.top_k, True)
+    wn = w.numpy()
+    EM = g["max_EM"]
+    eids16 = np.repeat(g["eids"], g["bs"] // 16).astype(np.int32)
+    oracle.set_act_model(1)
+    try:
+        c = cpu_layer(A, wn, ids, tw, threads=16)
+        partial = oracle.moe_down(g["act"], wn[2], wn[3], g["sids"], eids16, T, I, 0, I, H, cfg.top_k, EM)
+    finally:
+        oracle.set_act_model(0)
+    ref = oracle.moe_combine(partial, None, oracle.gather_sorted_weights(tw, g["sids"]), g["sids"], eids16, T, H,
+                             cfg.top_k, EM)
+    g_act, c_act = np.zeros((n_flat, I)), np.zeros((n_flat, I))
+    r = np.nonzero(g["sids"] < n_flat)[0]
+    g_act[g["sids"][r]] = synth.bf16_bits_to_f32(g["act"][r])
+    r = np.nonzero(c["sorted_ids"] < n_flat)[0]
+    c_act[c["sorted_ids"][r]] = synth.bf16_bits_to_f32(c["act"][r])
+    for p in np.unique(power):
+        t = np.nonzero(power == p)[0]
+        rows = (t[:, None] * cfg.top_k + np.arange(cfg.top_k)).ravel()
+        ga, ca = g_act[rows], c_act[rows]
+        assert np.all(np.isfinite(ga)) and np.all(np.isfinite(ca)), p
+        excess = np.abs(ga - ca) - (1e-3 * np.sqrt(np.mean(ca ** 2)) + 2.0 ** -7 * np.abs(ca))
+        assert float(excess.max()) <= 0.0, p
+        got, exp = g["out"][t].astype(np.float64), ref[t].astype(np.float64)
+        assert np.all(np.isfinite(got)) and np.all(np.isfinite(exp)), p
+        scale = np.sqrt(np.mean(exp ** 2))
+        if scale == 0.0:
+            assert not got.any(), p
+            continue
+        worst, rel = np.abs(got - exp).max() / scale, np.linalg.norm(got - exp) / np.linalg.norm(exp)
+        print(f"H={H} I={I} 2^{p}: max_abs/rms={worst:.3e} rel_l2={rel:.3e}")
+        assert worst <= EXACT_SPLIT_MAX_ABS_TOL and rel <= EXACT_SPLIT_REL_L2_TOL, p
