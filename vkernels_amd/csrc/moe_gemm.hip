@@ -2543,8 +2543,13 @@ __global__ __launch_bounds__(256) void fill_i32_kernel(int32_t* dst, int32_t val
 // nontemporal, here and where the prepacked second stage stores its rows.  Kept like other
 // lines they only throw out of the caches what is used again.  8191 tokens x 6 rows of 4096:
 // 205 -> 158 us here and 338 -> 324 us for the stage, 16384 x 8 of 7168: 856 -> 756 us and
-// 2563 -> 2461 us; whole layers 1.8 % (1400 x 6 rows of 4096, less than the last cache
-// holds) to 3.4 % (5500 x 6) faster, so no line is drawn by size.
+// 2563 -> 2461 us.  The combine of fewer rows is longer (1000 x 6 of 4096: 17.8 -> 20.4 us),
+// the layer is not: against ordinary stores and loads 207.0 -> 202.0 us for 300 x 6 of 4096,
+// 231.9 -> 225.0 for 500 x 6, 518 -> 506 for 1500 x 4 of 2880 with 128 experts, level for 300 to
+// 1000 x 4 of 2880 with 32, 409.4 -> 411.6 and 402 -> 405 us for 2048 x 4 of 2880 and 1500 x 6 of
+// 4096.  These two lie between sizes that gain, so no line is drawn by size.  A reader that
+// follows (the result added to a residual) makes no difference: 500 x 6 237.5 -> 232.7,
+// 2000 x 6 453.1 -> 454.3, 4000 x 6 846 -> 823 us with it.
 template <int TOPK>
 __global__ __launch_bounds__(256) void combine_kernel(const float* __restrict__ y,
                                                       const int32_t* __restrict__ pos,
