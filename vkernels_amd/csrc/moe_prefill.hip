@@ -290,10 +290,11 @@ __global__ __launch_bounds__(256) void split_rows_fp6_kernel(const uint16_t* __r
 // packed 16-bit integer operations on the bit patterns, which order like the magnitudes:
 // with z = (bits - bits(.125 x 2^(s-127)) + 32) / 32, clamped at zero, the thresholds
 // are z = 1, 10, 14, 16, 18, and the code is [z >= 1] + [z >= 10] + floor(max(z - 12, 0) / 2),
-// 8 instructions a value instead of the 20 of a chain of float comparisons.  Groups with a
-// NaN, or a scale so small or large that a threshold or a product leaves the normal
-// numbers (s outside 4 .. 143), take that chain.  4096 wide, 32768 sorted rows of which
-// 24576 routed: 72 -> 42 us.
+// 8 instructions a value instead of the 20 of a chain of float comparisons (13 with the group's
+// maximum, the scale byte and the addresses, by the counter).  Groups with a NaN, or a scale so
+// small or large that a threshold or a product leaves the normal numbers (s outside 4 .. 143),
+// take that chain.  4096 wide, 32768 sorted rows of which 24576 routed: 77 -> 46 us, 34 of them
+// the issue of the vector instructions.
 // ---------------------------------------------------------------------------
 typedef __attribute__((ext_vector_type(2))) uint16_t u16x2;
 
@@ -520,8 +521,8 @@ __global__ __launch_bounds__(256) void mxfp4_quant_kernel(const uint16_t* __rest
 // row, a block = the 32 codes moved onto the OCP code points (16 bytes), the scale byte
 // less one, 15 zero bytes; zero groups get a neutral scale.  row_bad[r] = 1 when a scale
 // byte is outside the range the scaled MFMA path takes.  8191 tokens x 6 rows of 1536:
-// 169 -> 59 us (4.1 TB/s) with as many rows a wavefront as it has lanes for (a workgroup per row left
-// four fifths of it idle) and the packed quantisation.
+// 171 -> 62 us (3.7 TB/s) with a wavefront per row (a workgroup per row, a group of 32 to a lane,
+// left four fifths of it idle), loads of a batch together and the packed quantisation.
 template <bool WIDE>
 __global__ __launch_bounds__(256) void quant_rows_w4_kernel(const uint16_t* __restrict__ x,
                                                             uint8_t* __restrict__ xq,

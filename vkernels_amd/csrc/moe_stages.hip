@@ -18,8 +18,9 @@ namespace {
 // act[r, c] = bf16(activation(gate_up[r, c] + b13[e, c], gate_up[r, ispp + c] + b13[e, ispp + c]))
 // for every routed sorted row r of a block with an expert (moe_act_epilogue_cpu,
 // src/c/vkernels/kernels/moe_fused.cpp:370-422); the other rows of act are left as they
-// are.  One thread per 4 columns.  The pre-activations are read once, past the caches (with the
-// stage kernels' stores of them: a rank of four's share of 2048 tokens 266.8 -> 262.6 us).
+// are.  One thread per 4 columns.  The pre-activations are read once, past the caches, as the
+// stage kernels store them (those stores: a rank of four's share of 2048 tokens 291 -> 281 us
+// in all).
 __global__ __launch_bounds__(256) void act_epilogue_kernel(
     const float* __restrict__ gate_up, const float* __restrict__ b13, uint16_t* __restrict__ act,
     const int32_t* __restrict__ sorted_ids, const int32_t* __restrict__ expert_ids, int n_flat, int EM,
