@@ -578,7 +578,7 @@ __global__ __launch_bounds__(256) void quant_rows_w4_kernel(const uint16_t* __re
 // tile t][activation row lane % 32] in the accumulator layout of the 32 x 32 MFMAs.
 // a_row: the bf16 row of this lane's activation row, or null for a padding row.
 // q_row (W4A4 mode): the row's quantised plane instead; its values are decoded exactly.
-template <int STAGE>
+template <bool ROWS_FIRST>
 __device__ __forceinline__ void exact_unit_mx(const MxArgs& p, int e, int unit, bool w_raw, const uint16_t* a_row,
                                               const uint8_t* q_row, int lane, f32x16 (&acc)[4]) {
   // The weights come from the packed form: K block g of row n of tile t is the 16 bytes
@@ -617,7 +617,10 @@ __device__ __forceinline__ void exact_unit_mx(const MxArgs& p, int e, int unit, 
         sc = (sc + 1u) & 0xFFu;
       }
       const u32x4 wv = dequant8_exact(c, sc);
-      acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(wv), as_bf16x8(av), acc[t], 0, 0, 0);
+      if constexpr (ROWS_FIRST)
+        acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(av), as_bf16x8(wv), acc[t], 0, 0, 0);
+      else
+        acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(wv), as_bf16x8(av), acc[t], 0, 0, 0);
     }
   }
 }
@@ -671,17 +674,18 @@ __device__ __forceinline__ i32x8 fp4_operand_ocp(u32x4 w) {  // codes already on
   return __builtin_shufflevector(y, y, 0, 1, 2, 3, -1, -1, -1, -1);
 }
 
-// One scaled MFMA: A = FP4 (cbsz 4) with scale byte T of wscale.  B = the operand read
-// from LDS: FP6 E2M3 (blgp 2, scale in byte 0 of b[6]) or, in the W4A4 mode, FP4 (blgp 4,
-// codes in b[0..3], scale in byte 0 of b[4]).
-template <int T, bool W4A4>
+// One scaled MFMA of the weights, FP4 with scale byte T of wscale, and the operand of rows read
+// from LDS: FP6 E2M3 (format 2, scale in byte 0 of b[6]) or, in the W4A4 mode, FP4 (format 4,
+// codes in b[0..3], scale in byte 0 of b[4]).  ROWS_FIRST: the rows as operand A and the weights
+// as B, so that a lane holds one column of 16 rows instead of 16 columns of one row.
+template <int T, bool W4A4, bool ROWS_FIRST>
 __device__ __forceinline__ f32x16 mfma_fp4_act(u32x4 w, i32x8 b, f32x16 acc, uint32_t wscale) {
-  if constexpr (W4A4)
-    return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fp4_operand_ocp(w), b, acc, 4, 4, T,
-                                                           (int)wscale, 0, b[4]);
+  if constexpr (ROWS_FIRST)
+    return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(b, fp4_operand_ocp(w), acc, W4A4 ? 4 : 2, 4, 0,
+                                                           b[W4A4 ? 4 : 6], T, (int)wscale);
   else
-    return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fp4_operand_ocp(w), b, acc, 4, 2, T,
-                                                           (int)wscale, 0, b[6]);
+    return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fp4_operand_ocp(w), b, acc, 4, W4A4 ? 4 : 2, T,
+                                                           (int)wscale, 0, b[W4A4 ? 4 : 6]);
 }
 
 // PREACT: the stage's linear part alone (tensor-parallel callers sum it over their K slices
@@ -689,13 +693,13 @@ __device__ __forceinline__ f32x16 mfma_fp4_act(u32x4 w, i32x8 b, f32x16 acc, uin
 // bias, no activation, no routing weight; rows that are not routed are left as they are.
 template <int STAGE, int TERMS, bool PREACT = false>
 __global__ __launch_bounds__(64 * kMxWaves) void tile_mx_kernel(MxArgs p) {
-  constexpr int R = kMxRing;
-  constexpr int kSlotBytes = kMxRows * TERMS * 128;
+  // fp32 rows leave straight from the accumulators (see the epilogue)
+  constexpr bool kRowsFirst = STAGE == 1 || PREACT;
   typedef __attribute__((address_space(3))) void* lds_ptr;
   extern __shared__ u32x4 mx_lds[];
   __shared__ int win_flat[kMxRows];  // sorted_ids of the window's rows, asked for before its experts are known
   __shared__ int row_flat[kMxRows];
-  __shared__ float row_w[kMxRows];  // stage 1: the routing weight of every row (0 where none is routed)
+  __shared__ alignas(16) float row_w[kMxRows];  // stage 1: the routing weight of every row (0 where none is routed)
   __shared__ int seg_hi[2];   // highest routed row index among rows 0..63 / 64..127 (or -1)
   __shared__ int seg_bad[2];  // a routed row of the half is outside the split's range
 
@@ -860,8 +864,7 @@ __global__ __launch_bounds__(64 * kMxWaves) void tile_mx_kernel(MxArgs p) {
     auto k_loop = [&](auto live_c) {
       constexpr int LIVE = decltype(live_c)::value;
       constexpr int Q = mx_step_groups(LIVE, TERMS);       // groups (operand reads) per step
-      constexpr int kPer = mx_ops_per_group(LIVE, TERMS);  // memory operations per issuing group
-      static_assert(Q >= 4 && kPer * (Q - 2) >= kOps, "a step's loads are all issued before its wait");
+      static_assert(Q >= 4 && mx_op_slot(LIVE, TERMS, kOps - 1) < 4 * (Q - 2), "a step's loads are all issued before its wait");
       auto group_operand = [&](const SlotBase& sb, int q) {
         return read_operand(sb, (q / TERMS) % LIVE, q % TERMS, q / (LIVE * TERMS));
       };
@@ -886,31 +889,35 @@ __global__ __launch_bounds__(64 * kMxWaves) void tile_mx_kernel(MxArgs p) {
         int slot_next = mx_ring_slot(c + 1);
         __asm__ volatile("" : "+s"(slot_next));
         const SlotBase sbn = slot_base(slot_next);
-        int issued = 0;
 #pragma unroll
         for (int q = 0; q < Q; ++q) {
           const int half = q / (LIVE * TERMS), m = (q / TERMS) % LIVE;
           const uint32_t wsc = ws[i].sc[half];
+          // the operations behind MFMA t of this group
+          auto issue_at = [&](int t) {
+#pragma unroll
+            for (int k = 0; k < kOps; ++k)
+              if (mx_op_slot(LIVE, TERMS, k) == 4 * q + t) issue(ws[in2], c + 2, k);
+          };
           // (a wavefront without a unit multiplies unit 0's weights and drops the result)
-          acc[m][0] = mfma_fp4_act<0, TERMS == 1>(ws[i].w[half * 4 + 0], cur, acc[m][0], wsc);
+          acc[m][0] = mfma_fp4_act<0, TERMS == 1, kRowsFirst>(ws[i].w[half * 4 + 0], cur, acc[m][0], wsc);
           __builtin_amdgcn_sched_barrier(0);
           // reads of group q + 2; the last two groups read the next step's first two
           const i32x8 pend = q + 2 < Q ? group_operand(sb, q + 2) : group_operand(sbn, q + 2 - Q);
+          issue_at(0);
           __builtin_amdgcn_sched_barrier(0);
-          acc[m][1] = mfma_fp4_act<1, TERMS == 1>(ws[i].w[half * 4 + 1], cur, acc[m][1], wsc);
+          acc[m][1] = mfma_fp4_act<1, TERMS == 1, kRowsFirst>(ws[i].w[half * 4 + 1], cur, acc[m][1], wsc);
           __builtin_amdgcn_sched_barrier(0);
-          if (q < Q - 2) {
-#pragma unroll
-            for (int k = 0; k < kPer; ++k)
-              if (issued + k < kOps) issue(ws[in2], c + 2, issued + k);
-            issued += kPer;
-          }
+          issue_at(1);
           __builtin_amdgcn_sched_barrier(0);
-          acc[m][2] = mfma_fp4_act<2, TERMS == 1>(ws[i].w[half * 4 + 2], cur, acc[m][2], wsc);
+          acc[m][2] = mfma_fp4_act<2, TERMS == 1, kRowsFirst>(ws[i].w[half * 4 + 2], cur, acc[m][2], wsc);
           __builtin_amdgcn_sched_barrier(0);
           __asm__ volatile("" : "+v"(nxt));  // complete from here on (read a group ago)
+          issue_at(2);
           __builtin_amdgcn_sched_barrier(0);
-          acc[m][3] = mfma_fp4_act<3, TERMS == 1>(ws[i].w[half * 4 + 3], cur, acc[m][3], wsc);
+          acc[m][3] = mfma_fp4_act<3, TERMS == 1, kRowsFirst>(ws[i].w[half * 4 + 3], cur, acc[m][3], wsc);
+          __builtin_amdgcn_sched_barrier(0);
+          issue_at(3);
           __builtin_amdgcn_sched_barrier(0);
           if (q == mx_wait_group(LIVE, TERMS)) {
             wait_loads_and_reads<kOps>(ws[in1]);
@@ -953,35 +960,41 @@ __global__ __launch_bounds__(64 * kMxWaves) void tile_mx_kernel(MxArgs p) {
     if (STAGE == 1 && !PREACT && colg == 0 && tid < n_rows && row_flat[tid] >= 0) p.pos[row_flat[tid]] = row0 + tid;
     if (!has_unit) return;
 
-    // ---- epilogue: lane (ln, hh) holds, of activation row 32 m + ln, the weight rows
-    // 8 (i / 4) + 4 hh + i % 4 of each tile: a few columns of 32 different rows.  Stored
-    // like that, every store instruction touches 64 cache lines; instead the values of 32
-    // rows go through a staging area of the wavefront's own in the ring (free after the
-    // barrier above) and leave as whole lines: 4 rows x 256 bytes (8 rows x 128 bytes in
-    // stage 0) per store instruction ----
+    // ---- epilogue.  fp32 rows (kRowsFirst): lane (ln, hh) holds, of column ln of each tile, rows
+    // 8 (i / 4) + 4 hh + i % 4 of the row tile; a store instruction writes two whole lines of 32
+    // columns, straight from the accumulators.  Without the way through LDS, and with the loop's
+    // loads spread evenly, the second stage of 16384 x 8 rows of 2048 x 7168 takes 2.39 instead of
+    // 2.50 ms, of 4096 x 4 of 2880 x 2880 245 instead of 260 us; of 1000 x 6 of 1536 x 4096 level.
+    // Activations (the same there is 1 to 3 % longer: arithmetic takes the time, not the stores):
+    // lane (ln, hh) holds, of row 32 m + ln, columns 8 (i / 4) + 4 hh + i % 4 of each tile; the
+    // values of 32 rows go through a staging area of the wavefront's own in the ring (free after
+    // the barrier above) and leave as whole lines, 8 rows x 128 bytes per store instruction ----
     uint8_t* stage_lds = reinterpret_cast<uint8_t*>(mx_lds) + mx_stage_base(wave, TERMS);
     auto wave_fence = [] {  // LDS operations of a wavefront execute in order; this keeps the compiler's too
       __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     };
-    // The biases of the columns this lane holds (the same for every row tile), tile by
-    // tile as the accumulators are laid out: asked for here, all at once, not value by
-    // value inside the loops below.
+    // The biases of the columns this lane holds (the same for every row tile): asked for here,
+    // all at once, not value by value inside the loops below.
     const bool has_bias = !PREACT && p.bias != nullptr;  // uniform
-    f32x4 bias_v[4][4];  // [tile][row group]
-    if (has_bias) {
-      // stage 0: tiles 0, 1 = gate columns, 2, 3 = the same columns of up
-      // stage 1: the last unit may be ragged (ncols is a multiple of 64); its columns past
-      // the end are not stored, so the first tiles' biases stand in
-      const float* b = p.bias + (STAGE == 0 ? (size_t)e * (size_t)(2 * p.ncols) + unit * 64
-                                            : (size_t)e * (size_t)p.ncols + unit * kMxUnitRows) + hh * 4;
+    float bias_c[4] = {0.f, 0.f, 0.f, 0.f};  // kRowsFirst: of the lane's column of each tile
+    f32x4 bias_v[4][4];                      // else [tile][row group]
+    if constexpr (kRowsFirst) {
+      if (has_bias) {
+        // (the last unit may be ragged (ncols is a multiple of 64); its columns past the end
+        // are not stored, so the first tiles' biases stand in)
+        const float* b = p.bias + (size_t)e * (size_t)p.ncols + unit * kMxUnitRows + ln;
 #pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const int c = STAGE == 0 ? (t >> 1) * p.ncols + (t & 1) * 32
-                                 : (unit * kMxUnitRows + (t >> 1) * 64 < p.ncols ? t * 32 : 0);
-#pragma unroll
-        for (int rg = 0; rg < 4; ++rg) bias_v[t][rg] = *reinterpret_cast<const f32x4u*>(b + c + rg * 8);
+        for (int t = 0; t < 4; ++t) bias_c[t] = b[unit * kMxUnitRows + (t >> 1) * 64 < p.ncols ? t * 32 : 0];
       }
-    } else if (STAGE == 0 && !PREACT && p.activation == 1) {  // the one loop that adds them without a bias
+    } else if (has_bias) {
+      // tiles 0, 1 = gate columns, 2, 3 = the same columns of up
+      const float* b = p.bias + (size_t)e * (size_t)(2 * p.ncols) + unit * 64 + hh * 4;
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int rg = 0; rg < 4; ++rg)
+          bias_v[t][rg] = *reinterpret_cast<const f32x4u*>(b + (t >> 1) * p.ncols + (t & 1) * 32 + rg * 8);
+    } else if (p.activation == 1) {  // the one loop that adds them without a bias
 #pragma unroll
       for (int i = 0; i < 16; ++i) bias_v[i >> 2][i & 3] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
@@ -1000,43 +1013,54 @@ __global__ __launch_bounds__(64 * kMxWaves) void tile_mx_kernel(MxArgs p) {
           if (TERMS == 1) q_row = p.Aq + grow * (size_t)Kp;
           else a_row = p.A + grow * (size_t)p.a_stride;
         }
-        exact_unit_mx<STAGE>(p, e, unit, w_slow, a_row, q_row, lane, tile);
+        exact_unit_mx<kRowsFirst>(p, e, unit, w_slow, a_row, q_row, lane, tile);
       }
-      if constexpr (PREACT) {
-        // the accumulators as they are: 64 columns (two tiles) at a time through the
-        // wavefront's staging area, whole lines out, routed rows only
-        // (nontemporal: read once, by the activation or the combine)
-        constexpr int kPitch = kMxYPitch;
-        const int width = STAGE == 0 ? 2 * p.ncols : p.ncols;
+      if constexpr (kRowsFirst) {
+        // (Nontemporal: the rows are read once, by combine_kernel, the activation or the combine
+        // of the stage split.)  In the second stage rows of the window that are not routed are
+        // stored like the others (with a routing weight of zero): nothing reads them (pos never
+        // points at them), and a later segment of this window, if they are its rows, overwrites
+        // them.  PREACT leaves them as they are.
+        uint32_t width = (uint32_t)(PREACT && STAGE == 0 ? 2 * p.ncols : p.ncols) * 4u;  // bytes of a row
+        __asm__ volatile("" : "+s"(width));  // (or the 16 rows' offsets are kept for the whole kernel)
+        char* const rows = reinterpret_cast<char*>(PREACT ? p.preact : p.y) + (size_t)(row0 + m * 32) * (size_t)width;  // uniform
+        const uint32_t lane_off = (uint32_t)(4 * hh) * width + 4u * (uint32_t)ln;
+        f32x4 w[4];  // routing weights (from LDS, put there when the rows were listed)
+        if constexpr (!PREACT) {
 #pragma unroll
-        for (int tp = 0; tp < 2; ++tp) {
-          // stage 0: tiles 0, 1 = gate columns of the unit, 2, 3 = the same columns of up
-          const int col0 = STAGE == 0 ? tp * p.ncols + unit * 64 : unit * kMxUnitRows + tp * 64;
-          if (STAGE == 1 && col0 >= p.ncols) break;  // uniform: the last unit may be ragged
-#pragma unroll
-          for (int tl = 0; tl < 2; ++tl)
-#pragma unroll
-            for (int rg = 0; rg < 4; ++rg) {
-              const int t = 2 * tp + tl;
-              const int cl = tl * 32 + rg * 8 + hh * 4;
-              *reinterpret_cast<f32x4*>(stage_lds + ln * kPitch + cl * 4) =
-                  f32x4{tile[t][rg * 4], tile[t][rg * 4 + 1], tile[t][rg * 4 + 2], tile[t][rg * 4 + 3]};
-            }
-          wave_fence();
-          f32x4 v[8];
-#pragma unroll
-          for (int pass = 0; pass < 8; ++pass)
-            v[pass] = *reinterpret_cast<const f32x4*>(stage_lds + (pass * 4 + (lane >> 4)) * kPitch + (lane & 15) * 16);
-          wave_fence();
-          float* dst = p.preact + (size_t)(row0 + m * 32 + (lane >> 4)) * (size_t)width + col0 + (lane & 15) * 4;
-#pragma unroll
-          for (int pass = 0; pass < 8; ++pass) {
-            if ((routed >> (pass * 4 + (lane >> 4))) & 1ull)
-              __builtin_nontemporal_store(v[pass], reinterpret_cast<f32x4*>(dst));
-            dst += 4 * (size_t)width;
-          }
+          for (int g = 0; g < 4; ++g) w[g] = *reinterpret_cast<const f32x4*>(row_w + m * 32 + 8 * g + 4 * hh);
         }
-      } else if (STAGE == 0) {
+        auto store_rows = [&](auto bias_k, auto guard_k) {
+          constexpr bool kBias = decltype(bias_k)::value != 0, kGuard = decltype(guard_k)::value != 0;
+#pragma unroll
+          for (int tp = 0; tp < 2; ++tp) {  // tiles 2 tp, 2 tp + 1
+            // stage 0: tiles 0, 1 = gate columns of the unit, 2, 3 = the same columns of up
+            const int col0 = STAGE == 0 ? tp * p.ncols + unit * 64 : unit * kMxUnitRows + tp * 64;
+            if (STAGE == 1 && col0 >= p.ncols) break;  // uniform: the last unit may be ragged (ncols is a multiple of 64)
+            char* dst = rows + (size_t)col0 * 4;  // uniform: of row 8 (i / 4) + i % 4
+#pragma unroll
+            for (int i = 0; i < 16; ++i, dst += (size_t)((i & 3) == 0 ? 5u : 1u) * (size_t)width) {
+              const int r = 8 * (i >> 2) + (i & 3);
+              if (kGuard && ((routed >> (r + 4 * hh)) & 1ull) == 0ull) continue;
+#pragma unroll
+              for (int tl = 0; tl < 2; ++tl) {
+                float v = tile[2 * tp + tl][i];
+                if constexpr (kBias) v += bias_c[2 * tp + tl];
+                if constexpr (!PREACT) v *= w[i >> 2][i & 3];
+                __builtin_nontemporal_store(v, reinterpret_cast<float*>(dst + lane_off) + tl * 32);
+              }
+            }
+          }
+        };
+        const bool whole = PREACT ? (uint32_t)routed == 0xFFFFFFFFu : row0 + m * 32 + 32 <= win_end;  // uniform
+        if (!has_bias) {
+          if (whole) store_rows(IntC<0>{}, IntC<0>{});
+          else store_rows(IntC<0>{}, IntC<1>{});
+        } else if constexpr (!PREACT) {
+          if (whole) store_rows(IntC<1>{}, IntC<0>{});
+          else store_rows(IntC<1>{}, IntC<1>{});
+        }
+      } else {
         constexpr int kPitch = kMxActPitch;
         // 128 activation values per lane and row tile.  A wavefront runs alone on its SIMD,
         // so a branch per value (bias or not, clamp or not, which activation) is paid in
@@ -1105,60 +1129,6 @@ __global__ __launch_bounds__(64 * kMxWaves) void tile_mx_kernel(MxArgs p) {
           if ((routed >> r) & 1ull)
             *reinterpret_cast<u32x4*>(p.act + (size_t)(row0 + m * 32 + r) * (size_t)p.ncols + unit * 64 +
                                       piece * 8) = v[pass];
-        }
-      } else {
-        // A wavefront runs alone on its SIMD, so every branch and every predicate of this
-        // code is paid in full; it is therefore specialised, per row tile, on what is
-        // uniform: a bias or none, and whether the tile's 32 rows all belong to this
-        // workgroup's window.  (Nontemporal stores: combine_kernel.)  Then rows that are not routed are stored like the others
-        // (with a routing weight of zero): nothing reads them (pos never points at them),
-        // and a later segment of this window, if they are its rows, overwrites them.
-        constexpr int kPitch = kMxYPitch;
-        // (from LDS, put there when the rows were listed: a load from memory still pending
-        // when the stores begin makes every later wait for it a wait for those stores)
-        const float w = row_w[m * 32 + ln];
-        auto store_rows = [&](auto bias_c, auto guard_c) {
-          constexpr bool kBias = decltype(bias_c)::value != 0, kGuard = decltype(guard_c)::value != 0;
-#pragma unroll
-          for (int tp = 0; tp < 2; ++tp) {  // tiles 2 tp, 2 tp + 1: 64 columns
-            const int col0 = unit * kMxUnitRows + tp * 64;
-            if (col0 >= p.ncols) break;  // uniform: the last unit may be ragged (ncols is a multiple of 64)
-#pragma unroll
-            for (int tl = 0; tl < 2; ++tl)
-#pragma unroll
-              for (int rg = 0; rg < 4; ++rg) {
-                const int t = 2 * tp + tl;
-                const int cl = tl * 32 + rg * 8 + hh * 4;
-                f32x4 v = {tile[t][rg * 4], tile[t][rg * 4 + 1], tile[t][rg * 4 + 2], tile[t][rg * 4 + 3]};
-                if constexpr (kBias) v += bias_v[t][rg];
-                *reinterpret_cast<f32x4*>(stage_lds + ln * kPitch + cl * 4) = v * w;
-              }
-            wave_fence();
-            f32x4 v[8];  // all the reads, one wait, then the stores: 4 rows x 256 bytes per instruction
-#pragma unroll
-            for (int pass = 0; pass < 8; ++pass)
-              v[pass] = *reinterpret_cast<const f32x4*>(stage_lds + (pass * 4 + (lane >> 4)) * kPitch + (lane & 15) * 16);
-            wave_fence();
-            float* dst = p.y + (size_t)(row0 + m * 32 + (lane >> 4)) * (size_t)p.ncols + col0 + (lane & 15) * 4;
-#pragma unroll
-            for (int pass = 0; pass < 8; ++pass) {
-              if constexpr (kGuard) {
-                if ((routed >> (pass * 4 + (lane >> 4))) & 1ull)
-                  __builtin_nontemporal_store(v[pass], reinterpret_cast<f32x4*>(dst));
-              } else {
-                __builtin_nontemporal_store(v[pass], reinterpret_cast<f32x4*>(dst));
-              }
-              dst += 4 * (size_t)p.ncols;
-            }
-          }
-        };
-        const bool inside = row0 + m * 32 + 32 <= win_end;  // uniform
-        if (!has_bias) {
-          if (inside) store_rows(IntC<0>{}, IntC<0>{});
-          else store_rows(IntC<0>{}, IntC<1>{});
-        } else {
-          if (inside) store_rows(IntC<1>{}, IntC<0>{});
-          else store_rows(IntC<1>{}, IntC<1>{});
         }
       }
     }

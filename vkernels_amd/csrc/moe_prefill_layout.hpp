@@ -111,12 +111,17 @@ __host__ __device__ constexpr inline int mx_ops_per_group(int live, int terms) {
   return (mx_step_ops(terms) + mx_step_groups(live, terms) - 3) / (mx_step_groups(live, terms) - 2);
 }
 __host__ __device__ constexpr inline int mx_wait_group(int live, int terms) { return mx_step_groups(live, terms) - 3; }
+// MFMA of the step that operation k is issued behind: evenly over those of groups 0 .. Q - 3
+// (never ahead of mx_ops_per_group a group, never behind group Q - 3)
+__host__ __device__ constexpr inline int mx_op_slot(int live, int terms, int k) {
+  return k * 4 * (mx_step_groups(live, terms) - 2) / mx_step_ops(terms);
+}
 
 // ---- epilogue staging: a wavefront's own quarter of the ring ----
 __host__ __device__ constexpr inline uint32_t mx_stage_base(int wave, int terms) {
   return (uint32_t)(wave * (kMxRing * mx_slot_bytes(terms) / kMxWaves));
 }
 constexpr int kMxActPitch = 144;  // stage 0: 64 bf16 of a row + 16 bytes (rows stay 16-byte aligned)
-constexpr int kMxYPitch = 272;    // stage 1: 64 floats of a row + 16 bytes
+constexpr int kMxYPitch = 272;    // 64 floats of a row + 16 bytes (room kept; fp32 rows are not staged)
 
 }  // namespace vk
