@@ -627,18 +627,28 @@ __device__ __forceinline__ void exact_unit_mx(const MxArgs& p, int e, int unit, 
 
 // Register load of 16 (8) bytes per lane at base + voff (+ an immediate), not
 // waited for: the caller counts it and passes the registers through wait_loads.
+// A memory operation may read a scalar register that a vector instruction wrote only five
+// wait states later, and the compiler, which keeps that distance otherwise, does not look
+// into inline assembly: where it brings a spilled base back (v_readlane) the operation
+// would take half of an old one.  So each goes through a copy of its base: a scalar
+// instruction may read the register at once, and the operation the copy.
 template <int OFF>
 __device__ __forceinline__ void load16_nowait(u32x4& dst, uint32_t voff, const uint8_t* base) {
-  __asm__ volatile("global_load_dwordx4 %0, %1, %2 offset:%3" : "=&v"(dst) : "v"(voff), "s"(base), "n"(OFF) : "memory");
+  uint64_t b;
+  __asm__ volatile("s_mov_b64 %1, %3\n\tglobal_load_dwordx4 %0, %2, %1 offset:%4"
+                   : "=&v"(dst), "=&s"(b) : "v"(voff), "s"(base), "n"(OFF) : "memory");
 }
 __device__ __forceinline__ void load8_nowait(u32x2& dst, uint32_t voff, const uint8_t* base) {
-  __asm__ volatile("global_load_dwordx2 %0, %1, %2" : "=&v"(dst) : "v"(voff), "s"(base) : "memory");
+  uint64_t b;
+  __asm__ volatile("s_mov_b64 %1, %3\n\tglobal_load_dwordx2 %0, %2, %1"
+                   : "=&v"(dst), "=&s"(b) : "v"(voff), "s"(base) : "memory");
 }
 // The DMA form with a uniform base and a 32-bit offset per lane: 16 bytes per lane to
-// LDS at lds_base + 16 * lane.
+// LDS at lds_base + 16 * lane.  (The copy of the base is also the wait state behind m0.)
 __device__ __forceinline__ void dma16_saddr(uint32_t voff, const uint8_t* base, uint32_t lds_base) {
-  __asm__ volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-                   :
+  uint64_t b;
+  __asm__ volatile("s_mov_b32 m0, %1\n\ts_mov_b64 %0, %3\n\tglobal_load_lds_dwordx4 %2, %0"
+                   : "=&s"(b)
                    : "s"(__builtin_amdgcn_readfirstlane(lds_base)), "v"(voff), "s"(base)
                    : "memory");
 }
