@@ -49,6 +49,9 @@ def _too_early(lines):
                     break
                 states += width
         width = int(operands[0], 0) + 1 if op == "s_nop" else 1
+        if re.match(r"s_(mov|add|sub|mul|lsh|ash|and|or|xor|min|max|cselect)", op) and operands:
+            for written, _ in history:  # (replaced by a scalar instruction: no distance to keep)
+                written -= _scalars(operands[0])
         history.append((_scalars(operands[0]) if op.startswith("v_") and operands else set(), width))
         history = history[-WAIT_STATES:]
     return found
@@ -60,6 +63,7 @@ def test_the_check_sees_a_load_that_comes_too_early():
     assert _too_early(code) == [("k", "global_load_dwordx4 v[74:77], v130, s[4:5]")]
     assert _too_early(code[:3] + ["  s_nop 4"] + code[3:]) == []
     assert _too_early(code[:3] + ["  s_nop 3"] + code[3:]) != []
+    assert _too_early(code[:3] + ["  s_mov_b64 s[4:5], s[8:9]"] + code[3:]) == []
 
 
 @pytest.mark.parametrize("unit", ["moe_prefill", "moe_gemm"])

@@ -1,0 +1,87 @@
+"""The prefill kernels on the raw tensors: their loads, lane offsets and K loop's schedule walked on
+the CPU (tests/prefill_raw_layout_check.cpp), and on the GPU against the same call on prepacked
+weights with three terms in both stages, which multiplies and adds the same values in the same
+order: the same bits, whatever the window, the epilogue or the path of a unit."""
+from __future__ import annotations
+
+import subprocess
+import sys
+from pathlib import Path
+
+import pytest
+import torch
+
+ROOT = Path(__file__).resolve().parents[1]
+sys.path.insert(0, str(ROOT))
+from vkernels_amd import vllm_experts as ve  # noqa: E402
+
+
+def _build(tmp_path, *defines):
+    exe = tmp_path / "prefill_raw_layout_check"
+    subprocess.run(["g++", "-O2", "-std=c++17", "-Wall", "-Werror", *defines, f"-I{ROOT / 'vkernels_amd' / 'csrc'}",
+                    str(ROOT / "tests" / "prefill_raw_layout_check.cpp"), "-o", str(exe)], check=True)
+    return exe
+
+
+def test_offsets_and_schedule(tmp_path):
+    exe = _build(tmp_path)
+    for args in ("0 7168 2048 3", "1 2048 7168 3", "0 4096 1536 2", "1 1536 4096 2", "0 512 512 2", "1 512 512 2"):
+        res = subprocess.run([str(exe), *args.split()], capture_output=True, text=True)
+        assert res.returncode == 0, f"{args}: {res.stderr.strip()}"
+
+
+@pytest.mark.parametrize("wait", [0, 1])
+def test_the_walk_notices_a_wait_that_counts_wrong(tmp_path, wait):
+    exe = _build(tmp_path, f"-DVK_LAYOUT_BREAK_WAIT={wait}")
+    assert subprocess.run([str(exe), "0", "7168", "2048", "3"], capture_output=True).returncode == 1
+
+
+def _weights(E, H, I, gen, special):
+    def codes(*shape):
+        c = torch.randint(0, 256, shape, dtype=torch.uint8, device="cuda", generator=gen)
+        finite = c & ~((((c >> 1) & c) & 0x22) << 1)     # codes 6 and 7 of either sign become 2 and 3
+        return finite
+    def scales(*shape):
+        return torch.randint(120, 131, shape, dtype=torch.uint8, device="cuda", generator=gen)
+    w = [codes(E, 2 * I, H // 2), scales(E, 2 * I, H // 32), codes(E, H, I // 2), scales(E, H, I // 32)]
+    if special:  # units that take the exact path: an infinity, a NaN, scale bytes at and past the range's ends
+        w[0][0, 3, 5] = 0x06
+        w[2][E - 1, H - 1, I // 2 - 1] = 0x70
+        w[1][1, 2 * I - 1, H // 32 - 1] = 63
+        w[1][1, 70, 0] = 64
+        w[3][1, 200, 3] = 191
+        w[3][2, 130, 1] = 190
+    return w
+
+
+# rows a block of 50 on, and rounds of workgroups that are not nearly empty (the call's own rule);
+# H, I multiples of 512: the shortest loops (4 K steps), windows of 1 to 4 live row tiles
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,I,E,k,T,epilogue,special", [
+    (512, 512, 4, 2, 9999, "plain", False), (512, 512, 4, 2, 10111, "clamp", True),
+    (1024, 512, 60, 4, 3000, "situ", False), (1024, 1536, 16, 2, 7001, "plain", True),
+    (4096, 1536, 64, 6, 1100, "clamp", False),
+])
+def test_same_bits_as_on_prepacked_weights(H, I, E, k, T, epilogue, special):
+    gen = torch.Generator(device="cuda").manual_seed(T)
+    w = _weights(E, H, I, gen, special)
+    kw = {}
+    if epilogue != "plain":
+        kw = dict(b13=torch.randn((E, 2 * I), device="cuda", generator=gen),
+                  b2=torch.randn((E, H), device="cuda", generator=gen))
+        kw.update(dict(swiglu_limit=7.0) if epilogue == "clamp" else dict(activation="situ", beta=3.0, linear_beta=20.0))
+    A = torch.randn((T, H), device="cuda", generator=gen).to(torch.bfloat16)
+    if special:
+        A[5, 7], A[T - 1, H - 1] = float("inf"), 1e-38   # rows outside the range of the split
+    logits = torch.randn((T, E), device="cuda", generator=gen)
+    raw = ve.FusedExperts(*w, **kw)
+    packed = ve.FusedExperts(*w, prepack=True, split_terms=3, **kw)
+    ids, tw = raw.route(logits, k)
+    assert raw.block_size_for(T, k) == 128
+    a = raw.apply(A, ids, tw, output_dtype=torch.float32)
+    b = packed.apply(A, ids, tw, output_dtype=torch.float32)
+    assert torch.equal(torch.isnan(a), torch.isnan(b))
+    assert torch.equal(torch.nan_to_num(a), torch.nan_to_num(b))
+    # ... and the raw call is not the slower kernels' (their two FP8 terms round differently)
+    again = raw.apply(A, ids, tw, output_dtype=torch.float32)
+    assert torch.equal(torch.nan_to_num(a), torch.nan_to_num(again))

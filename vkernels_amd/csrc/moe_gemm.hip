@@ -3191,6 +3191,7 @@ void launch_moe_down(const FusedMoeArgs& a, hipStream_t stream) {
   const bool overwrite = (a.flags & 1u) != 0u;  // VK_HIP_MOE_OVERWRITE_OUT
   if (pl.variant != kMoeVariantResident) {
     if (a.w2_packed != nullptr && launch_moe_down_prepacked(a, stream)) return;
+    if (launch_moe_down_prepacked(a, stream, true)) return;
     Workspace w;
     if (carve_workspace(a, w) && g.K >= 512 && wide_kernel_ready<1>()) {
       const long long pieces = (long long)a.EM * split_row_k(a.ispp) / 8;
@@ -3230,6 +3231,10 @@ void launch_fused_moe(const FusedMoeArgs& a, hipStream_t stream) {
     (void)launch_fused_moe_prepacked(a, stream);
     return;
   }
+  // ... and the same kernels on the raw tensors where they take them
+  if (p0.variant != kMoeVariantResident && p1.variant != kMoeVariantResident &&
+      launch_fused_moe_prepacked(a, stream, true))
+    return;
   Workspace w;
   bool combine = false;
   bool split_act_between = false;

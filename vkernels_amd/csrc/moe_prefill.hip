@@ -78,6 +78,8 @@ typedef __attribute__((ext_vector_type(32))) __bf16 bf16x32;
 struct MxArgs {
   const uint8_t* Wp;       // prepacked weights of the stage
   const uint8_t* Wflags;   // [E, units]: 1 = the unit takes the exact path
+  const uint8_t* W;        // RAW: codes and scale bytes as the checkpoint has them
+  const uint8_t* Ws;
   const uint16_t* A;       // bf16 rows (exact path): stage 0 A [M, K], stage 1 act [EM, K]
   const uint8_t* Aq;       // split rows: row r = TERMS planes of Kp bytes at r * TERMS * Kp
   const uint8_t* row_bad;  // per row of Aq: 1 = outside the split's range
@@ -578,7 +580,7 @@ __global__ __launch_bounds__(256) void quant_rows_w4_kernel(const uint16_t* __re
 // tile t][activation row lane % 32] in the accumulator layout of the 32 x 32 MFMAs.
 // a_row: the bf16 row of this lane's activation row, or null for a padding row.
 // q_row (W4A4 mode): the row's quantised plane instead; its values are decoded exactly.
-template <bool ROWS_FIRST>
+template <int STAGE, bool ROWS_FIRST, bool RAW>
 __device__ __forceinline__ void exact_unit_mx(const MxArgs& p, int e, int unit, bool w_raw, const uint16_t* a_row,
                                               const uint8_t* q_row, int lane, f32x16 (&acc)[4]) {
   // The weights come from the packed form: K block g of row n of tile t is the 16 bytes
@@ -586,7 +588,9 @@ __device__ __forceinline__ void exact_unit_mx(const MxArgs& p, int e, int unit, 
   // for (half, t) of that lane's eight.  A flagged unit (w_raw) holds the codes and
   // scale bytes of the raw tensors; any other the codes moved onto the OCP points and
   // the scale bytes less one, both undone here (all its codes are finite).
-  const int n = lane & 31, hh = lane >> 5;
+  int n = lane & 31;
+  const int hh = lane >> 5;
+  if (RAW) __asm__ volatile("" : "+v"(n));  // (or the rows' offsets are kept in registers through the K loop)
   const int K = p.K;
   const int nsteps = mx_kp(K) / 128;
   const uint8_t* const ub = p.Wp + mx_unit_offset(e, p.units, unit, nsteps);
@@ -610,9 +614,17 @@ __device__ __forceinline__ void exact_unit_mx(const MxArgs& p, int e, int unit, 
     const int half = (g >> 1) & 1, lane_p = (g & 1) * 32 + n;
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
-      uint32_t c = *reinterpret_cast<const uint32_t*>(sb + half * 4096 + t * 1024 + lane_p * 16 + ((k & 31) >> 1));
-      uint32_t sc = sb[8192 + lane_p * 8 + half * 4 + t];
-      if (!w_raw) {
+      uint32_t c, sc;
+      if constexpr (RAW) {
+        const int rows = STAGE == 0 ? 2 * p.ncols : p.ncols;
+        const size_t row = (size_t)e * rows + mx_raw_row(STAGE, p.ncols, unit, t, n);
+        c = *reinterpret_cast<const uint32_t*>(p.W + row * (size_t)(K / 2) + (size_t)(k >> 1));
+        sc = p.Ws[row * (size_t)(K / 32) + g];
+      } else {
+        c = *reinterpret_cast<const uint32_t*>(sb + half * 4096 + t * 1024 + lane_p * 16 + ((k & 31) >> 1));
+        sc = sb[8192 + lane_p * 8 + half * 4 + t];
+      }
+      if (!RAW && !w_raw) {
         c -= (c & 0x44444444u) >> 1;
         sc = (sc + 1u) & 0xFFu;
       }
@@ -651,6 +663,32 @@ __device__ __forceinline__ void dma16_saddr(uint32_t voff, const uint8_t* base, 
                    : "=&s"(b)
                    : "s"(__builtin_amdgcn_readfirstlane(lds_base)), "v"(voff), "s"(base)
                    : "memory");
+}
+
+// The same in all lanes (mask ~0) or in none (0; uniform), without a branch: one in the K loop makes
+// the register allocator shuffle accumulators.
+__device__ __forceinline__ void dma16_masked(uint32_t mask, uint32_t voff, const uint8_t* base, uint32_t lds_base) {
+  uint64_t exec, b;
+  __asm__ volatile("s_mov_b64 %0, exec\n\ts_mov_b32 exec_lo, %5\n\ts_mov_b32 exec_hi, %5\n\ts_mov_b32 m0, %2\n\t"
+                   "s_mov_b64 %1, %4\n\tglobal_load_lds_dwordx4 %3, %1\n\ts_mov_b64 exec, %0"
+                   : "=&s"(exec), "=&s"(b)
+                   : "s"(__builtin_amdgcn_readfirstlane(lds_base)), "v"(voff), "s"(base),
+                     "s"(__builtin_amdgcn_readfirstlane(mask))
+                   : "memory");
+}
+
+struct WeightHalf {  // half a K step of a unit in registers, raw codes
+  u32x4 w[4];        // [tile]
+};
+
+// As wait_loads below, for half a step; and for the wavefront's LDS reads as well.
+template <int N>
+__device__ __forceinline__ void wait_half(WeightHalf& h) {
+  __asm__ volatile("s_waitcnt vmcnt(%[n])" : "+v"(h.w[0]), "+v"(h.w[1]), "+v"(h.w[2]), "+v"(h.w[3]) : [n] "n"(N) : "memory");
+}
+template <int N>
+__device__ __forceinline__ void wait_half_and_reads(WeightHalf& h) {
+  __asm__ volatile("s_waitcnt vmcnt(%[n]) lgkmcnt(0)" : "+v"(h.w[0]), "+v"(h.w[1]), "+v"(h.w[2]), "+v"(h.w[3]) : [n] "n"(N) : "memory");
 }
 
 struct WeightStep {  // one K step of a unit in registers
@@ -701,7 +739,18 @@ __device__ __forceinline__ f32x16 mfma_fp4_act(u32x4 w, i32x8 b, f32x16 acc, uin
 // PREACT: the stage's linear part alone (tensor-parallel callers sum it over their K slices
 // before the epilogue): the accumulators of the routed rows go to p.preact as fp32, no
 // bias, no activation, no routing weight; rows that are not routed are left as they are.
-template <int STAGE, int TERMS, bool PREACT = false>
+// f(IntC<0>), ..., f(IntC<N - 1>): indices that are constants before anything is unrolled.
+template <int N, int I = 0, typename F>
+__device__ __forceinline__ void static_for(F f) {
+  if constexpr (I < N) {
+    f(IntC<I>{});
+    static_for<N, I + 1>(f);
+  }
+}
+
+// RAW: the weights as the checkpoint has them (p.W, p.Ws), moved onto the code points and checked
+// in the loop.
+template <int STAGE, int TERMS, bool PREACT = false, bool RAW = false>
 __global__ __launch_bounds__(64 * kMxWaves) void tile_mx_kernel(MxArgs p) {
   // fp32 rows leave straight from the accumulators (see the epilogue)
   constexpr bool kRowsFirst = STAGE == 1 || PREACT;
@@ -777,7 +826,8 @@ __global__ __launch_bounds__(64 * kMxWaves) void tile_mx_kernel(MxArgs p) {
     const int hi = seg_hi[1] >= 0 ? 64 + seg_hi[1] : seg_hi[0];
     const int n_live = (hi + 32) >> 5;  // row tiles of 32 up to the last routed row
     if (n_live == 0) return;            // uniform
-    const bool w_slow = has_unit && p.Wflags[(size_t)e * p.units + unit] != 0;  // uniform per wavefront
+    bool w_slow = false;  // uniform per wavefront
+    if constexpr (!RAW) w_slow = has_unit && p.Wflags[(size_t)e * p.units + unit] != 0;
 
     // ---- row copies: one instruction moves 8 rows x 128 bytes of one term.  Lane
     // (r, c) = (lane / 8, lane % 8) copies piece c ^ r of its row, so LDS position c of
@@ -954,8 +1004,167 @@ __global__ __launch_bounds__(64 * kMxWaves) void tile_mx_kernel(MxArgs p) {
       wait_loads<0>(ws[1]);
       wait_loads<0>(ws[2]);
     };
+    // The same on raw weights.  A lane's 16 bytes lie in a line of their own, so an operand load
+    // occupies the memory pipe 75 cycles instead of 18 (measured, 4 wavefronts): 8 of them, the
+    // row copies and the scale bytes are 3.3 k cycles a step of 3.1 k cycles of MFMAs, whatever
+    // the live rows.  4096 tokens of 256 experts of 7168 x 2048: 2622 -> 2190 us this stage and
+    // 1412 -> 1280 us the second against tile_wide_kernel; 64 experts of 4096 x 1536: 774 -> 585
+    // and 452 -> 350 us.  (Loads of 16 rows x 64 bytes, 37 cycles each, put in order by a lane
+    // permutation through LDS and row swaps, were 1 to 4 % behind at these sizes and ahead where
+    // this form is not taken.)
+    auto raw_loop = [&](auto live_c) {
+      constexpr int LIVE = decltype(live_c)::value;
+      constexpr int G = mx_raw_groups(LIVE, TERMS), Q = 2 * G, kHalfOps = mx_raw_ops(TERMS);
+      static_assert(G >= 3 && mx_raw_fix_slot(LIVE, TERMS, 15) < 4 * G, "the waits and the code points");
+      const int rows_w = STAGE == 0 ? 2 * p.ncols : p.ncols;
+      const uint8_t* const w_base = p.W + (size_t)e * (size_t)rows_w * (size_t)(K / 2);
+      const uint8_t* const s_base = p.Ws + (size_t)e * (size_t)rows_w * (size_t)(K / 32);
+      uint32_t w_off[4], s_off[2];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) w_off[t] = mx_raw_lane_offset(mx_raw_row(STAGE, p.ncols, unit, t, ln), K, hh);
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        s_off[i] = (uint32_t)mx_raw_row(STAGE, p.ncols, unit, 2 * i + hh, ln) * (uint32_t)(K / 32);
+      const uint32_t s_lds = (uint32_t)(kMxRing * mx_slot_bytes(TERMS) + wave * kMxRawScaleBytes);
+      auto copy_scales = [&](int step, uint32_t mask) {  // of steps step .. step + 3
+        const uint8_t* src = s_base + 4 * min(step, nsteps - 4);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) dma16_masked(mask, s_off[i], src, lds_base + s_lds + 1024u * i);
+      };
+      uint32_t bad = 0u;
+      // scale bytes of a step, less one: byte 0 / 2 = this lane's K block of half 0 / 1 of tile t
+      struct StepScales {
+        uint32_t t[4];
+      };
+      auto read_scales = [&](int step) {
+        StepScales r;
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+          r.t[t] = *reinterpret_cast<const uint32_t*>(lds_bytes + s_lds + (32 * t + ln) * 16 + (step & 3) * 4);
+        return r;
+      };
+      static_assert(kScaleLo == 64u && kScaleHi == 190u, "the check of ready_scales");
+      auto ready_scales = [&](StepScales& r) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          // a byte outside [64, 190]: neither of its two top bits is set, or both are in it or in
+          // the byte plus one
+          const uint32_t v = r.t[t], v1 = v + 0x01010101u;
+          bad |= (~(v | (v << 1)) | (v & (v << 1)) | (v1 & (v1 << 1))) & 0x80808080u;
+          r.t[t] = (v - 0x01010101u) >> (8 * hh);
+        }
+      };
+      // the operands on the code points, of half 0 and half 1 (words of their own, not the load's
+      // registers rewritten: the register allocator would move whole tuples about)
+      uint32_t fx[2][4][4];
+      auto fix_word = [&](uint32_t& dst, uint32_t w) {
+        bad |= fp4x8_nonfinite(w);
+        dst = fp4x8_to_ocp_doubled(w);
+      };
+      // operation k (0 .. kHalfOps - 1) of a half step, for half step `half` of K step `step`
+      auto issue_raw = [&](WeightHalf& h, int step, int half, int k) {
+        if (k < 4) load16_nowait<0>(h.w[k], w_off[k], w_base + mx_raw_load_offset(step, nsteps, half));
+        else copy_rows(step, half * (kHalfOps - 4) + k - 4);
+      };
+      auto base_of = [&](int slot_) {
+        uint32_t off = rd_off[0] + (uint32_t)(slot_ * mx_slot_bytes(TERMS));
+        __asm__ volatile("" : "+v"(off));
+        return off;
+      };
+      // (the pieces of a K block are 16, 64 and 80 bytes off by exclusive or)
+      auto group_operand = [&](uint32_t base, int q) {
+        const int half = q / (LIVE * TERMS);
+        const int tile_off = (int)mx_operand_tile_offset(0, TERMS, (q / TERMS) % LIVE, q % TERMS);
+        const u32x4 lo = *reinterpret_cast<const u32x4*>(lds_bytes + (base ^ (64u * half)) + tile_off);
+        const u32x4 hi4 = *reinterpret_cast<const u32x4*>(lds_bytes + (base ^ (64u * half + 16u)) + tile_off);
+        return i32x8{(int)lo[0], (int)lo[1], (int)lo[2], (int)lo[3],
+                     (int)hi4[0], (int)hi4[1], (int)hi4[2], (int)hi4[3]};
+      };
+      WeightHalf hs[4];
+      copy_scales(0, ~0u);
+      static_for<4>([&](auto s_c) {
+#pragma unroll
+        for (int k = 0; k < kHalfOps; ++k) issue_raw(hs[decltype(s_c)::value], decltype(s_c)::value >> 1, decltype(s_c)::value & 1, k);
+      });
+      wait_half<2 * kHalfOps>(hs[0]);
+      wait_half<2 * kHalfOps>(hs[1]);
+      __builtin_amdgcn_s_barrier();
+      __asm__ volatile("" ::: "memory");
+      StepScales sc = read_scales(0), sc_next;
+      ready_scales(sc);
+      static_for<16>([&](auto x_c) {
+        constexpr int x = decltype(x_c)::value;
+        fix_word(fx[0][x >> 2][x & 3], hs[0].w[x >> 2][x & 3]);
+      });
+      uint32_t sb = base_of(0);
+      i32x8 cur = group_operand(sb, 0);
+      i32x8 nxt = group_operand(sb, 1);
+
+      auto step = [&](auto i_c, const int c) {  // i = c % 2 picks the register sets
+        constexpr int i = decltype(i_c)::value;
+        int slot_next = mx_ring_slot(c + 1);
+        __asm__ volatile("" : "+s"(slot_next));
+        const uint32_t sbn = base_of(slot_next);
+        static_for<Q>([&](auto q_c) {
+          constexpr int q = decltype(q_c)::value;
+          constexpr int half = q / G, m = (q / TERMS) % LIVE;
+          i32x8 pend;
+          static_for<4>([&](auto t_c) {
+            constexpr int t = decltype(t_c)::value;
+            const u32x4 w = {fx[half][t][0], fx[half][t][1], fx[half][t][2], fx[half][t][3]};
+            acc[m][t] = mfma_fp4_act<2 * half, false, kRowsFirst>(w, cur, acc[m][t], sc.t[t]);
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (t == 0) pend = q + 2 < Q ? group_operand(sb, q + 2) : group_operand(sbn, q + 2 - Q);
+            if constexpr (t == 2) __asm__ volatile("" : "+v"(nxt));  // complete from here on (read a group ago)
+            static_for<kHalfOps>([&](auto k_c) {
+              if constexpr (mx_raw_op_slot(LIVE, TERMS, decltype(k_c)::value) == 4 * (q - half * G) + t)
+                issue_raw(hs[mx_raw_weight_set(2 * i + half)], c + 2, half, decltype(k_c)::value);
+            });
+            static_for<16>([&](auto x_c) {
+              constexpr int x = decltype(x_c)::value;
+              if constexpr (mx_raw_fix_slot(LIVE, TERMS, x) == 4 * (q - half * G) + t)
+                fix_word(fx[half ^ 1][x >> 2][x & 3], hs[mx_raw_weight_set(2 * i + half + 1)].w[x >> 2][x & 3]);
+            });
+            __builtin_amdgcn_sched_barrier(0);
+          });
+          if constexpr (q == G - 1) {  // the middle of the step
+            wait_half<mx_raw_middle_wait(LIVE, TERMS)>(hs[mx_raw_weight_set(2 * i + 2)]);
+            sc_next = read_scales(c + 1);  // (behind the last step: bytes of it again, not used)
+            __builtin_amdgcn_sched_barrier(0);
+          }
+          if constexpr (q == G) {
+            ready_scales(sc_next);  // (its reads are complete, so their bytes may be replaced)
+            __builtin_amdgcn_sched_barrier(0);
+            copy_scales(c + 2, (uint32_t)-(int)((c & 3) == 2 && c + 2 < nsteps));
+            __builtin_amdgcn_sched_barrier(0);
+          }
+          if constexpr (q == Q - 3) {
+            wait_half_and_reads<mx_raw_row_wait(LIVE, TERMS)>(hs[mx_raw_weight_set(2 * i + 3)]);
+            __builtin_amdgcn_s_barrier();
+            __asm__ volatile("" ::: "memory");
+          }
+          cur = nxt;
+          nxt = pend;
+        });
+        sb = sbn;
+        sc = sc_next;
+      };
+#pragma unroll 1
+      for (int c0 = 0; c0 < nsteps; c0 += 2) {  // (nsteps is a multiple of four)
+        step(IntC<0>{}, c0);
+        step(IntC<1>{}, c0 + 1);
+      }
+      // the loads issued past the last step write registers and the ring: let them land
+#pragma unroll
+      for (int j = 0; j < 4; ++j) wait_half<0>(hs[j]);
+      w_slow = has_unit && __ballot(bad != 0u) != 0ull;
+    };
     // (one plane per row: a step of one row tile would be shorter than the pipeline)
-    if (n_live > 3) k_loop(IntC<4>{});
+    if constexpr (RAW) {
+      if (n_live > 3) raw_loop(IntC<4>{});
+      else if (n_live == 3) raw_loop(IntC<3>{});
+      else raw_loop(IntC<2>{});  // (one row tile takes as long: the loads bound both)
+    } else if (n_live > 3) k_loop(IntC<4>{});
     else if (n_live == 3) k_loop(IntC<3>{});
     else if (n_live == 2 || TERMS == 1) k_loop(IntC<2>{});
     else if constexpr (TERMS > 1) k_loop(IntC<1>{});
@@ -1023,7 +1232,7 @@ __global__ __launch_bounds__(64 * kMxWaves) void tile_mx_kernel(MxArgs p) {
           if (TERMS == 1) q_row = p.Aq + grow * (size_t)Kp;
           else a_row = p.A + grow * (size_t)p.a_stride;
         }
-        exact_unit_mx<kRowsFirst>(p, e, unit, w_slow, a_row, q_row, lane, tile);
+        exact_unit_mx<STAGE, kRowsFirst, RAW>(p, e, unit, w_slow, a_row, q_row, lane, tile);
       }
       if constexpr (kRowsFirst) {
         // (Nontemporal: the rows are read once, by combine_kernel, the activation or the combine
@@ -1161,19 +1370,24 @@ __global__ __launch_bounds__(64 * kMxWaves) void tile_mx_kernel(MxArgs p) {
   }
 }
 
-template <int STAGE, int TERMS, bool PREACT = false>
+template <int TERMS, bool RAW>
+constexpr int mx_lds_bytes() {
+  return kMxRing * mx_slot_bytes(TERMS) + (RAW ? kMxWaves * kMxRawScaleBytes : 0);
+}
+
+template <int STAGE, int TERMS, bool PREACT = false, bool RAW = false>
 bool mx_kernel_ready() {
   static const bool configured = [] {
     const hipError_t err = hipFuncSetAttribute(
-        reinterpret_cast<const void*>(tile_mx_kernel<STAGE, TERMS, PREACT>),
-        hipFuncAttributeMaxDynamicSharedMemorySize, kMxRing * kMxRows * TERMS * 128);
+        reinterpret_cast<const void*>(tile_mx_kernel<STAGE, TERMS, PREACT, RAW>),
+        hipFuncAttributeMaxDynamicSharedMemorySize, mx_lds_bytes<TERMS, RAW>());
     if (err != hipSuccess) (void)hipGetLastError();  // not left for the next caller to find
     return err == hipSuccess;
   }();
   return configured;
 }
 
-template <int STAGE, int TERMS, bool PREACT = false>
+template <int STAGE, int TERMS, bool PREACT = false, bool RAW = false>
 void launch_mx_stage_t(MxArgs g, hipStream_t stream) {
   const int win = mx_window_rows(g.block_size);
   g.units = mx_units(STAGE, g.ncols);
@@ -1181,8 +1395,8 @@ void launch_mx_stage_t(MxArgs g, hipStream_t stream) {
   g.windows = (g.num_blocks * g.block_size + win - 1) / win;
   const long long total = (long long)g.col_groups * g.windows;
   const unsigned grid = (unsigned)((total + 255) / 256 * 256);  // whole chunks of 32 tiles for each of 8 XCDs
-  hipLaunchKernelGGL((tile_mx_kernel<STAGE, TERMS, PREACT>), dim3(grid), dim3(64 * kMxWaves),
-                     kMxRing * kMxRows * TERMS * 128, stream, g);
+  hipLaunchKernelGGL((tile_mx_kernel<STAGE, TERMS, PREACT, RAW>), dim3(grid), dim3(64 * kMxWaves),
+                     (mx_lds_bytes<TERMS, RAW>()), stream, g);
 }
 
 MxArgs mx_args(const FusedMoeArgs& a, int stage) {
@@ -1262,7 +1476,7 @@ bool prepare_mx_kernels() {
   return mx_kernel_ready<0, 1>() && mx_kernel_ready<0, 2>() && mx_kernel_ready<0, 3>() &&
          mx_kernel_ready<1, 1>() && mx_kernel_ready<1, 2>() && mx_kernel_ready<1, 3>() &&
          mx_kernel_ready<0, 2, true>() && mx_kernel_ready<0, 3, true>() && mx_kernel_ready<1, 2, true>() &&
-         mx_kernel_ready<1, 3, true>();
+         mx_kernel_ready<1, 3, true>() && mx_kernel_ready<0, 3, false, true>() && mx_kernel_ready<1, 3, false, true>();
 }
 
 namespace {
@@ -1277,13 +1491,48 @@ struct MxPlan {
   // FP6 terms per activation in the first and in the second stage (2 or 3), or 1 and 1 =
   // the W4A4 mode (MXFP4 activations)
   int terms0, terms1;
+  bool raw;  // on the raw tensors, three terms in both stages
 };
 
-// False when the prepacked path does not take the call (no packed weights, workspace
+// Weights of one stage that the raw form of the kernels takes (mx_raw_* in moe_prefill_layout.hpp).
+bool mx_raw_takes(const uint8_t* w, const uint8_t* w_scale, int rows, int K) {
+  return w != nullptr && w_scale != nullptr && (reinterpret_cast<uintptr_t>(w) & 15) == 0 &&
+         (reinterpret_cast<uintptr_t>(w_scale) & 15) == 0 && K % kMxRawK == 0 && rows % 64 == 0 &&
+         (unsigned long long)rows * (unsigned long long)(K / 2) < (1ull << 32);
+}
+
+// Where the raw form is ahead of tile_wide_kernel: many rows for the blocks they are in, as each
+// window costs the raw loads whatever its rows (a whole layer, apply, tile_wide -> raw: 8 rows a
+// block of 64 experts 233 -> 294 us, 35 298 -> 330, 44 340 -> 351, 55 397 -> 389, 77 753 -> 584, 96
+// 1310 -> 1089; of 256 experts 26 2045 -> 2153, 43 2557 -> 2438, 64 4157 -> 3803), and no round of
+// workgroups of twice tile_wide's columns that is nearly empty (8 experts of 4096 x 4096, 4000 rows,
+// second stage 280 workgroups for 256 compute units: 530 -> 548 us).  The number of experts is not
+// known here: the padding of the sorted order is 127 rows for each of them, half a window in use.
+constexpr int kMxRawRows = 50;
+bool mx_raw_pays(const FusedMoeArgs& a) {
+  const long long rows = (long long)a.M * a.top_k;
+  if (rows * kMxRows < (long long)kMxRawRows * a.EM) return false;
+  const long long windows = rows / kMxRows + (a.EM - rows) / (2 * (kMxRows - 1)) + 1;
+  for (int stage = 0; stage < 2; ++stage) {
+    const int units = mx_units(stage, stage == 0 ? a.ispp : a.hidden);
+    const long long tiles = windows * ((units + kMxWaves - 1) / kMxWaves);
+    if (5 * tiles < 3 * ((tiles + 255) / 256 * 256)) return false;
+  }
+  return true;
+}
+
+// False when the path does not take the call (no weights in its form, workspace
 // short or misaligned, split rows beyond the 32-bit offsets of the row copies, LDS refused).
-bool mx_plan(const FusedMoeArgs& a, bool need_stage0, MxPlan& pl) {
-  if ((need_stage0 && a.w13_packed == nullptr) || a.w2_packed == nullptr || a.workspace == nullptr)
+bool mx_plan(const FusedMoeArgs& a, bool need_stage0, bool raw, MxPlan& pl) {
+  if (a.workspace == nullptr) return false;
+  if (raw) {
+    if (!mx_raw_pays(a) || (need_stage0 && !mx_raw_takes(a.w13, a.w13_scale, 2 * a.ispp, a.hidden)) ||
+        !mx_raw_takes(a.w2, a.w2_scale, a.hidden, a.ispp) || a.ispp % 64 != 0)
+      return false;
+  } else if ((need_stage0 && a.w13_packed == nullptr) || a.w2_packed == nullptr) {
     return false;
+  }
+  pl.raw = raw;
   const MxWorkspace l = mx_workspace(a.M, a.hidden, a.ispp, a.top_k, a.EM);
   if (a.workspace_bytes < l.total() || (reinterpret_cast<uintptr_t>(a.workspace) & 15) != 0) return false;
   if ((unsigned long long)a.EM * 3ull * mx_kp(a.ispp) >= (1ull << 32) ||
@@ -1295,13 +1544,20 @@ bool mx_plan(const FusedMoeArgs& a, bool need_stage0, MxPlan& pl) {
   // grows as the sums get shorter (1.7e-2 of the RMS at ispp = 64, 6.7e-3 at 256,
   // 4.6e-3 at 1024 and beyond with two terms; 2.5e-4 at 64 with three), and such
   // layers are small enough that the third term costs microseconds
-  if ((a.flags & 4u) != 0u) pl.terms0 = pl.terms1 = 1;
+  // On the raw tensors three in both: no further from the layer in 64 bits than the two FP8 terms
+  // of the kernels that take such calls where this path does not (8.5e-5 against 1.36e-4 for 1100
+  // tokens of 64 experts of 4096 x 1536, 8.3e-5 against 1.40e-4 for 4096 of 256 of 7168 x 2048,
+  // 5.7e-5 against 9.1e-5 for 3000 of 60 of 1024 x 512, bias and clamp).
+  if (raw) pl.terms0 = pl.terms1 = 3;
+  else if ((a.flags & 4u) != 0u) pl.terms0 = pl.terms1 = 1;
   else if ((a.flags & 2u) != 0u) pl.terms0 = pl.terms1 = 2;
   else if ((a.flags & 8u) != 0u) pl.terms0 = pl.terms1 = 3;
   else { pl.terms0 = 3; pl.terms1 = a.ispp < kMxShortK ? 3 : 2; }
-  const bool ready0 = !need_stage0 || (pl.terms0 == 1 ? mx_kernel_ready<0, 1>()
+  const bool ready0 = !need_stage0 || (raw ? mx_kernel_ready<0, 3, false, true>()
+                                       : pl.terms0 == 1 ? mx_kernel_ready<0, 1>()
                                        : pl.terms0 == 2 ? mx_kernel_ready<0, 2>() : mx_kernel_ready<0, 3>());
-  const bool ready1 = pl.terms1 == 1 ? mx_kernel_ready<1, 1>()
+  const bool ready1 = raw ? mx_kernel_ready<1, 3, false, true>()
+                      : pl.terms1 == 1 ? mx_kernel_ready<1, 1>()
                       : pl.terms1 == 2 ? mx_kernel_ready<1, 2>() : mx_kernel_ready<1, 3>();
   if (!ready0 || !ready1) return false;
   uint8_t* base = static_cast<uint8_t*>(a.workspace);
@@ -1313,12 +1569,19 @@ bool mx_plan(const FusedMoeArgs& a, bool need_stage0, MxPlan& pl) {
   pl.pos = reinterpret_cast<int32_t*>(pl.cbad + l.cbad + l.y);
   pl.g0 = mx_args(a, 0);
   pl.g1 = mx_args(a, 1);
-  const int units0 = mx_units(0, a.ispp), units1 = mx_units(1, a.hidden);
-  pl.g0.Wp = a.w13_packed;
-  pl.g0.Wflags = a.w13_packed == nullptr ? nullptr :
-      a.w13_packed + mx_packed_body_bytes(a.num_experts, units0, mx_kp(a.hidden) / 128);
-  pl.g1.Wp = a.w2_packed;
-  pl.g1.Wflags = a.w2_packed + mx_packed_body_bytes(a.num_experts, units1, mx_kp(a.ispp) / 128);
+  if (raw) {
+    pl.g0.W = a.w13;
+    pl.g0.Ws = a.w13_scale;
+    pl.g1.W = a.w2;
+    pl.g1.Ws = a.w2_scale;
+  } else {
+    const int units0 = mx_units(0, a.ispp), units1 = mx_units(1, a.hidden);
+    pl.g0.Wp = a.w13_packed;
+    pl.g0.Wflags = a.w13_packed == nullptr ? nullptr :
+        a.w13_packed + mx_packed_body_bytes(a.num_experts, units0, mx_kp(a.hidden) / 128);
+    pl.g1.Wp = a.w2_packed;
+    pl.g1.Wflags = a.w2_packed + mx_packed_body_bytes(a.num_experts, units1, mx_kp(a.ispp) / 128);
+  }
   pl.g0.Aq = pl.aq; pl.g0.row_bad = pl.abad;
   pl.g1.Aq = pl.cq; pl.g1.row_bad = pl.cbad;
   pl.g1.y = pl.y; pl.g1.pos = pl.pos;
@@ -1346,7 +1609,8 @@ void mx_stage0(const FusedMoeArgs& a, const MxPlan& pl, hipStream_t stream) {
     launch_mx_stage_t<0, 2>(pl.g0, stream);
   } else {
     hipLaunchKernelGGL(split_rows_fp6_kernel<3>, split_grid(a.M, a.hidden), dim3(256), 0, stream, a.A, pl.aq, pl.abad, a.hidden, a.hidden, a.M, nullptr, 0, nullptr, 0);
-    launch_mx_stage_t<0, 3>(pl.g0, stream);
+    if (pl.raw) launch_mx_stage_t<0, 3, false, true>(pl.g0, stream);
+    else launch_mx_stage_t<0, 3>(pl.g0, stream);
   }
 }
 
@@ -1362,34 +1626,35 @@ void mx_stage1(const FusedMoeArgs& a, const MxPlan& pl, hipStream_t stream) {
     launch_mx_stage_t<1, 2>(pl.g1, stream);
   } else {
     hipLaunchKernelGGL(split_rows_fp6_kernel<3>, split_grid(a.EM, a.ispp), dim3(256), 0, stream, a.act, pl.cq, pl.cbad, a.ispp, a.ispp, a.EM, a.sorted_ids, a.M * a.top_k, pl.pos, a.M * a.top_k);
-    launch_mx_stage_t<1, 3>(pl.g1, stream);
+    if (pl.raw) launch_mx_stage_t<1, 3, false, true>(pl.g1, stream);
+    else launch_mx_stage_t<1, 3>(pl.g1, stream);
   }
   launch_combine(pl.y, pl.pos, a.out, a.M, a.top_k, a.hidden, (a.flags & 1u) != 0u, stream);
 }
 
 }  // namespace
 
-// The whole layer on prepacked weights; false when the path does not take the call
-// (nothing has been enqueued then).
-bool launch_fused_moe_prepacked(const FusedMoeArgs& a, hipStream_t stream) {
+// The whole layer on prepacked weights, or on the raw tensors; false when the path does not
+// take the call (nothing has been enqueued then).
+bool launch_fused_moe_prepacked(const FusedMoeArgs& a, hipStream_t stream, bool raw) {
   MxPlan pl;
-  if (!mx_plan(a, true, pl)) return false;
+  if (!mx_plan(a, true, raw, pl)) return false;
   mx_stage0(a, pl, stream);
   mx_stage1(a, pl, stream);
   return true;
 }
 
 // True when launch_fused_moe_prepacked (both_stages) or launch_moe_down_prepacked would
-// take the call (nothing is enqueued).
+// take the call on prepacked weights (nothing is enqueued).
 bool fused_moe_prepacked_takes(const FusedMoeArgs& a, bool both_stages) {
   MxPlan pl;
-  return mx_plan(a, both_stages, pl);
+  return mx_plan(a, both_stages, false, pl);
 }
 
 // The second stage alone (act is the caller's), likewise.
-bool launch_moe_down_prepacked(const FusedMoeArgs& a, hipStream_t stream) {
+bool launch_moe_down_prepacked(const FusedMoeArgs& a, hipStream_t stream, bool raw) {
   MxPlan pl;
-  if (!mx_plan(a, false, pl)) return false;
+  if (!mx_plan(a, false, raw, pl)) return false;
   mx_stage1(a, pl, stream);
   return true;
 }

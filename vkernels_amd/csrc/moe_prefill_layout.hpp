@@ -117,6 +117,56 @@ __host__ __device__ constexpr inline int mx_op_slot(int live, int terms, int k) 
   return k * 4 * (mx_step_groups(live, terms) - 2) / mx_step_ops(terms);
 }
 
+// ---- raw weights: [E][rows][K / 2] codes and [E][rows][K / 32] scale bytes, as the checkpoint has
+// them.  K is a multiple of 512, so that four K steps of a row's scale bytes are 16 aligned bytes.
+// A unit is the 128 weight rows it is above; lane (n, hh) of operand load (half, t) takes the 16
+// bytes of K block 2 half + hh of row (t, n) itself. ----
+constexpr int kMxRawK = 512;
+__host__ __device__ constexpr inline int mx_raw_row(int stage, int ncols, int unit, int t, int n) {
+  const int row = mx_weight_row(stage, ncols, unit, t, n), rows = stage == 0 ? 2 * ncols : ncols;
+  return row < rows ? row : rows - 1;  // (stage 1's last unit may be ragged)
+}
+__host__ __device__ constexpr inline uint32_t mx_raw_lane_offset(int row, int K, int hh) {
+  return (uint32_t)row * (uint32_t)(K / 2) + 16u * (uint32_t)hh;
+}
+// (a step past the end: the last one again)
+__host__ __device__ constexpr inline uint32_t mx_raw_load_offset(int step, int nsteps, int half) {
+  return (uint32_t)((step < nsteps - 1 ? step : nsteps - 1) * 64 + half * 32);
+}
+// Scale bytes come to a wavefront's own 2 KiB of LDS, 16 of each of its 128 rows at a time.
+constexpr int kMxRawScaleBytes = 2048;
+// The K loop.  K step c is the half steps 2c, 2c + 1 (the halves of its operand tiles), each with
+// half of the row copies.  Half step s multiplies the operands that half step s - 1 has moved onto
+// the OCP code points, moves those of s + 1, and issues the 4 weight loads of s + 4, into the
+// registers whose codes half step s - 1 has moved, then its part of the row copies of K step
+// c + 2, spread evenly.  The scale bytes of step c + 1 are read from LDS in the middle of step c;
+// behind the first group after the middle of the last but one step of four the two copies for the
+// next four are issued (masked off in the other steps).
+__host__ __device__ constexpr inline int mx_raw_weight_set(int half_step) { return half_step & 3; }
+__host__ __device__ constexpr inline int mx_raw_ops(int terms) { return 4 + mx_row_ops(terms) / 2; }  // of a half step
+__host__ __device__ constexpr inline int mx_raw_groups(int live, int terms) { return live * terms; }  // of a half step
+__host__ __device__ constexpr inline int mx_raw_op_slot(int live, int terms, int k) {  // MFMA it follows
+  return k * 4 * mx_raw_groups(live, terms) / mx_raw_ops(terms);
+}
+// operations of a half step that are issued by the end of its group g
+__host__ __device__ constexpr inline int mx_raw_ops_through(int live, int terms, int g) {
+  int n = 0;
+  for (int k = 0; k < mx_raw_ops(terms); ++k) n += mx_raw_op_slot(live, terms, k) < 4 * (g + 1) ? 1 : 0;
+  return n;
+}
+// Waits (operations that may be outstanding).  In the middle of a step: those that have followed
+// the scale bytes' copies of the step before, which covers the weights the second half step moves
+// (three half steps old).  Before the barrier, behind the last group but two, the rows of step
+// c + 1 have landed and the weights that its first half step moves: all but the step's own.
+__host__ __device__ constexpr inline int mx_raw_middle_wait(int live, int terms) {
+  return 2 * mx_raw_ops(terms) - mx_raw_ops_through(live, terms, 0);
+}
+__host__ __device__ constexpr inline int mx_raw_row_wait(int live, int terms) {
+  return mx_raw_ops(terms) + mx_raw_ops_through(live, terms, mx_raw_groups(live, terms) - 3);
+}
+// MFMA of a half step behind which word w (0 .. 15) of the other half is moved onto the code points
+__host__ __device__ constexpr inline int mx_raw_fix_slot(int live, int terms, int w) { return w * live * terms / 4; }
+
 // ---- epilogue staging: a wavefront's own quarter of the ring ----
 __host__ __device__ constexpr inline uint32_t mx_stage_base(int wave, int terms) {
   return (uint32_t)(wave * (kMxRing * mx_slot_bytes(terms) / kMxWaves));
