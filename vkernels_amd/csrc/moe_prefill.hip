@@ -51,6 +51,8 @@
 //     sits between them.
 // All loads are issued by inline assembly and waited for with counted
 // s_waitcnt, because each wavefront issues them in a fixed order.
+// The RAW form of the kernel reads the weights as the checkpoint has them, for callers
+// that do not prepack; its loads, lane order and schedule are raw_loop's.
 //
 // Workgroup ids are mapped to (window, unit group) so that the 32 workgroups
 // resident on one XCD at a time cover 4 windows x 8 unit groups or the like:
