@@ -54,7 +54,7 @@ struct Event {
 // Program order of the K loop and what follows it, as tile_mx_kernel issues it.
 std::vector<Event> schedule(int terms, int live, int nsteps) {
   const int ops = mx_step_ops(terms), rows = mx_row_ops(terms);
-  const int Q = mx_step_groups(live, terms), per = mx_ops_per_group(live, terms);
+  const int Q = mx_step_groups(live, terms);
   std::vector<Event> ev;
   auto issue = [&](int step, int k) { ev.push_back({k < rows ? Event::kCopy : Event::kLoad, step, 0}); };
   // prologue: the operations of steps 0 and 1, a wait that leaves step 1's outstanding, a barrier,
@@ -70,14 +70,12 @@ std::vector<Event> schedule(int terms, int live, int nsteps) {
   ev.push_back({Event::kRead, 0, 0});
   ev.push_back({Event::kRead, 0, 0});
   for (int c = 0; c < nsteps; ++c) {
-    int issued = 0;
     for (int q = 0; q < Q; ++q) {
-      ev.push_back({Event::kUse, c, 0});                                     // the group's MFMAs
-      ev.push_back({Event::kRead, q + 2 < Q ? c : c + 1, 0});                // the operand of group q + 2
-      if (q < Q - 2) {
-        for (int k = 0; k < per; ++k)
-          if (issued + k < ops) issue(c + 2, issued + k);
-        issued += per;
+      for (int t = 0; t < 4; ++t) {
+        ev.push_back({Event::kUse, c, 0});                                   // MFMA t of the group
+        if (t == 0) ev.push_back({Event::kRead, q + 2 < Q ? c : c + 1, 0});  // the operand of group q + 2
+        for (int k = 0; k < ops; ++k)                                        // what is issued behind it
+          if (mx_op_slot(live, terms, k) == 4 * q + t) issue(c + 2, k);
       }
       if (q == mx_wait_group(live, terms)) {
         ev.push_back({Event::kWait, c, ops});
@@ -99,7 +97,7 @@ int check_schedule(int terms, int live, int nsteps) {
   std::vector<int> vm;          // issue positions (indices into ev) of the vector-memory operations, in order
   size_t landed = 0;            // operations known to have landed (a wait forced them)
   // per K step: operations issued, operations landed, landed-and-behind-a-barrier (every wavefront's),
-  // reads issued, reads completed, completed-and-behind-a-barrier, MFMA groups issued
+  // reads issued, reads completed, completed-and-behind-a-barrier, MFMAs issued
   const int S = nsteps + 4;
   std::vector<int> issued(S, 0), done(S, 0), done_all(S, 0), reads(S, 0), reads_done(S, 0), reads_done_all(S, 0), uses(S, 0);
   std::vector<int> step_of;     // step of each vector-memory operation
@@ -123,7 +121,7 @@ int check_schedule(int terms, int live, int nsteps) {
       case Event::kLoad: {
         const int old = e.step - 3;  // the register set's previous step: its MFMAs are all issued
         if (old >= 0 && old < nsteps)
-          CHECK(uses[old] == mx_step_groups(live, terms), "terms %d live %d nsteps %d: a weight load of step %d is "
+          CHECK(uses[old] == 4 * mx_step_groups(live, terms), "terms %d live %d nsteps %d: a weight load of step %d is "
                 "issued before the MFMAs of step %d", terms, live, nsteps, e.step, old);
         CHECK(mx_weight_set(e.step) == mx_weight_set(e.step + 3), "sets");
         vm.push_back((int)i);
@@ -167,8 +165,8 @@ int check_schedule(int terms, int live, int nsteps) {
     }
   }
   // every K step was multiplied, with all its groups, and every step's operations were issued once
-  for (int c = 0; c < nsteps; ++c) CHECK(uses[c] == mx_step_groups(live, terms) && issued[c] == ops, "step %d", c);
-  CHECK(mx_ops_per_group(live, terms) * (mx_step_groups(live, terms) - 2) >= ops, "a step's operations do not fit its groups");
+  for (int c = 0; c < nsteps + 2; ++c)
+    CHECK(uses[c] == (c < nsteps ? 4 * mx_step_groups(live, terms) : 0) && issued[c] == ops, "step %d", c);
   return 0;
 }
 
@@ -265,14 +263,14 @@ int main(int argc, char** argv) {
             }
           }
   }
-  // ---- epilogue staging ----
-  for (int wave = 0; wave < kMxWaves; ++wave) {
+  // ---- epilogue staging (the first stage's activations; fp32 rows are not staged) ----
+  for (int wave = 0; stage == 0 && wave < kMxWaves; ++wave) {
     const int lo = (int)mx_stage_base(wave, terms);
     const int hi = wave + 1 < kMxWaves ? (int)mx_stage_base(wave + 1, terms) : ring;
-    const int need = stage == 0 ? 31 * kMxActPitch + 128 : 31 * kMxYPitch + 256;
+    const int need = 31 * kMxActPitch + 128;
     CHECK(lo % 16 == 0 && lo + need <= hi, "staging area of wavefront %d: %d bytes in [%d, %d)", wave, need, lo, hi);
   }
-  CHECK(kMxActPitch % 16 == 0 && kMxYPitch % 16 == 0, "pitch");
+  CHECK(kMxActPitch % 16 == 0, "pitch");
   // ---- the K loop's schedule: every number of live row tiles the kernel compiles, the
   // problem's own K steps and the shortest loops ----
   for (int live = 1; live <= 4; ++live) {

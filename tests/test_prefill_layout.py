@@ -72,3 +72,20 @@ def test_the_checker_notices_a_wait_that_counts_wrong(tmp_path):
                     str(ROOT / "tests" / "prefill_layout_check.cpp"), "-o", str(exe)], check=True)
     res = subprocess.run([str(exe), "1", "2", "2048", "7168", "4", "640"], capture_output=True, text=True)
     assert res.returncode == 1 and "before every wavefront's copies of it have landed" in res.stderr
+
+
+@pytest.mark.parametrize("slot", ["4 * mx_step_groups(live, terms) - 1",                                 # behind the wait
+                                  "k + 1 < mx_step_ops(terms) ? 0 : 4 * (mx_step_groups(live, terms) - 2)",  # the last one is
+                                  "k == 0 ? -1 : 0"])                                                      # one never issued
+def test_the_checker_notices_an_operation_out_of_place(tmp_path, slot):
+    """The walk issues by mx_op_slot, as the kernel does: copies of the header in which it names
+    another MFMA are flagged, whichever operation is out of place."""
+    src = (ROOT / "vkernels_amd" / "csrc" / "moe_prefill_layout.hpp").read_text()
+    slots = "return k * 4 * (mx_step_groups(live, terms) - 2) / mx_step_ops(terms);"
+    assert src.count(slots) == 1
+    (tmp_path / "moe_prefill_layout.hpp").write_text(src.replace(slots, f"return {slot};"))
+    exe = tmp_path / "broken_slot"
+    subprocess.run(["g++", "-O2", "-std=c++17", f"-I{tmp_path}", str(ROOT / "tests" / "prefill_layout_check.cpp"),
+                    "-o", str(exe)], check=True)
+    res = subprocess.run([str(exe), "1", "2", "2048", "7168", "4", "640"], capture_output=True, text=True)
+    assert res.returncode == 1 and "FAILED" in res.stderr

@@ -104,15 +104,11 @@ __host__ __device__ constexpr inline int mx_row_ops(int terms) { return 4 * term
 __host__ __device__ constexpr inline int mx_step_ops(int terms) { return mx_row_ops(terms) + 9; }
 // groups of 4 MFMAs (one operand read each) per K step with `live` row tiles
 __host__ __device__ constexpr inline int mx_step_groups(int live, int terms) { return 2 * live * terms; }
-// The operations of step c + 2 are issued in groups 0 .. Q - 3 of step c, this many per
-// group; the step's one wait (at most mx_step_ops outstanding: step c + 1 has landed, step
-// c + 2 may be on its way) and barrier come at the end of group Q - 3.
-__host__ __device__ constexpr inline int mx_ops_per_group(int live, int terms) {
-  return (mx_step_ops(terms) + mx_step_groups(live, terms) - 3) / (mx_step_groups(live, terms) - 2);
-}
+// The step's one wait (at most mx_step_ops outstanding: step c + 1 has landed, step c + 2 may be
+// on its way) and barrier come at the end of group Q - 3.
 __host__ __device__ constexpr inline int mx_wait_group(int live, int terms) { return mx_step_groups(live, terms) - 3; }
-// MFMA of the step that operation k is issued behind: evenly over those of groups 0 .. Q - 3
-// (never ahead of mx_ops_per_group a group, never behind group Q - 3)
+// MFMA of step c (4 q + t: the t-th of group q) that operation k of step c + 2 is issued behind:
+// evenly over the MFMAs of groups 0 .. Q - 3, so that all of them are ahead of the wait
 __host__ __device__ constexpr inline int mx_op_slot(int live, int terms, int k) {
   return k * 4 * (mx_step_groups(live, terms) - 2) / mx_step_ops(terms);
 }
@@ -172,6 +168,5 @@ __host__ __device__ constexpr inline uint32_t mx_stage_base(int wave, int terms)
   return (uint32_t)(wave * (kMxRing * mx_slot_bytes(terms) / kMxWaves));
 }
 constexpr int kMxActPitch = 144;  // stage 0: 64 bf16 of a row + 16 bytes (rows stay 16-byte aligned)
-constexpr int kMxYPitch = 272;    // 64 floats of a row + 16 bytes (room kept; fp32 rows are not staged)
 
 }  // namespace vk
