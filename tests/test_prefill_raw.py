@@ -4,6 +4,7 @@ weights with three terms in both stages, which multiplies and adds the same valu
 order: the same bits, whatever the window, the epilogue or the path of a unit."""
 from __future__ import annotations
 
+import ctypes
 import subprocess
 import sys
 from pathlib import Path
@@ -34,6 +35,44 @@ def test_offsets_and_schedule(tmp_path):
 def test_the_walk_notices_a_wait_that_counts_wrong(tmp_path, wait):
     exe = _build(tmp_path, f"-DVK_LAYOUT_BREAK_WAIT={wait}")
     assert subprocess.run([str(exe), "0", "7168", "2048", "3"], capture_output=True).returncode == 1
+
+
+@pytest.fixture(scope="module")
+def raw_rule(tmp_path_factory):
+    """mx_raw_pays (moe_prefill_layout.hpp), compiled for the host: rows, EM, block, ispp, hidden -> taken?"""
+    d = tmp_path_factory.mktemp("rule")
+    (d / "rule.cpp").write_text('''#include "moe_prefill_layout.hpp"
+extern "C" int pays(long long r, long long em, int b, int i, int h) { return vk::mx_raw_pays(r, em, b, i, h); }''')
+    subprocess.run(["g++", "-O1", "-std=c++17", "-Wall", "-Werror", "-shared", "-fPIC",
+                    f"-I{ROOT / 'vkernels_amd' / 'csrc'}", str(d / "rule.cpp"), "-o", str(d / "rule.so")], check=True)
+    fn = ctypes.CDLL(str(d / "rule.so")).pays
+    fn.argtypes = [ctypes.c_longlong, ctypes.c_longlong, ctypes.c_int, ctypes.c_int, ctypes.c_int]
+    return fn
+
+
+@pytest.mark.parametrize("H,I,E,k", [(7168, 2048, 256, 8), (4096, 1536, 64, 6), (1024, 512, 60, 4)])
+@pytest.mark.parametrize("block,refused,taken", [
+    # rows an expert: the raw form was measured behind at all the first, ahead at the second where
+    # its rounds of workgroups are not nearly empty
+    (16, (12, 24, 36, 64, 96), 192), (32, (12, 24, 36, 64, 96), 192), (64, (12, 24, 36, 48), 192),
+    (128, (12, 24, 36, 48, 64), 192), (48, (12, 24, 36), 192), (80, (24, 36), 192), (96, (24, 36), 192), (112, (24, 36), 192),
+])
+def test_few_rows_a_segment_are_left_to_the_other_kernel(raw_rule, H, I, E, k, block, refused, taken):
+    for rows in refused:
+        T = rows * E // k
+        assert not raw_rule(T * k, ve._align_em_bound(T, k, E, block), block, I, H), rows
+        assert not raw_rule(T * k, (T * k + block - 1) // block * block + E * block, block, I, H), rows
+    T = taken * E // k
+    assert raw_rule(T * k, ve._align_em_bound(T, k, E, block), block, I, H)
+
+
+@pytest.mark.parametrize("block", [16, 48, 64, 128, 256])
+def test_the_rule_takes_any_sizes(raw_rule, block):
+    """... of a valid call: EM below the rows (an expert map drops the others), or far above."""
+    for rows in (1, 513, 8192, 2 ** 31 - 1):
+        for em in (block, rows // 2 // block * block + block, 2 ** 31 - 1):
+            for width in (64, 512, 7168):
+                assert raw_rule(rows, em, block, width, width) in (0, 1)
 
 
 def _weights(E, H, I, gen, special):

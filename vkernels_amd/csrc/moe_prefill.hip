@@ -1520,32 +1520,12 @@ bool mx_raw_takes(const uint8_t* w, const uint8_t* w_scale, int rows, int K) {
          (unsigned long long)rows * (unsigned long long)(K / 2) < (1ull << 32);
 }
 
-// Where the raw form is ahead of tile_wide_kernel: many rows for the blocks they are in, as each
-// window costs the raw loads whatever its rows (a whole layer, apply, tile_wide -> raw: 8 rows a
-// block of 64 experts 233 -> 294 us, 35 298 -> 330, 44 340 -> 351, 55 397 -> 389, 77 753 -> 584, 96
-// 1310 -> 1089; of 256 experts 26 2045 -> 2153, 43 2557 -> 2438, 64 4157 -> 3803), and no round of
-// workgroups of twice tile_wide's columns that is nearly empty (8 experts of 4096 x 4096, 4000 rows,
-// second stage 280 workgroups for 256 compute units: 530 -> 548 us).  The number of experts is not
-// known here: the padding of the sorted order is 127 rows for each of them, half a window in use.
-constexpr int kMxRawRows = 50;
-bool mx_raw_pays(const FusedMoeArgs& a) {
-  const long long rows = (long long)a.M * a.top_k;
-  if (rows * kMxRows < (long long)kMxRawRows * a.EM) return false;
-  const long long windows = rows / kMxRows + (a.EM - rows) / (2 * (kMxRows - 1)) + 1;
-  for (int stage = 0; stage < 2; ++stage) {
-    const int units = mx_units(stage, stage == 0 ? a.ispp : a.hidden);
-    const long long tiles = windows * ((units + kMxWaves - 1) / kMxWaves);
-    if (5 * tiles < 3 * ((tiles + 255) / 256 * 256)) return false;
-  }
-  return true;
-}
-
 // False when the path does not take the call (no weights in its form, workspace
 // short or misaligned, split rows beyond the 32-bit offsets of the row copies, LDS refused).
 bool mx_plan(const FusedMoeArgs& a, bool need_stage0, bool raw, MxPlan& pl) {
   if (a.workspace == nullptr) return false;
   if (raw) {
-    if (!mx_raw_pays(a) || (need_stage0 && !mx_raw_takes(a.w13, a.w13_scale, 2 * a.ispp, a.hidden)) ||
+    if (!mx_raw_pays((long long)a.M * a.top_k, a.EM, a.block_size, a.ispp, a.hidden) || (need_stage0 && !mx_raw_takes(a.w13, a.w13_scale, 2 * a.ispp, a.hidden)) ||
         !mx_raw_takes(a.w2, a.w2_scale, a.hidden, a.ispp) || a.ispp % 64 != 0)
       return false;
   } else if ((need_stage0 && a.w13_packed == nullptr) || a.w2_packed == nullptr) {

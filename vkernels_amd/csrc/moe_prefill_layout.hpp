@@ -163,6 +163,46 @@ __host__ __device__ constexpr inline int mx_raw_row_wait(int live, int terms) {
 // MFMA of a half step behind which word w (0 .. 15) of the other half is moved onto the code points
 __host__ __device__ constexpr inline int mx_raw_fix_slot(int live, int terms, int w) { return w * live * terms / 4; }
 
+// Where the raw form is ahead of tile_wide_kernel: many rows for the segments (the rows of one
+// expert in a window) they are in, as each segment costs the raw loads whatever its rows.  The number
+// of experts is not known here: EM is taken for the bound the sorted order is allocated by, block_size
+// - 1 rows of padding for each expert, half of it in use.  (An EM of the padded rows themselves makes
+// the experts half as many: calls up to a tenth behind are then taken too.)  Figures: a whole layer,
+// tile_wide -> raw.
+//   Blocks of 128 and more: 50 rows a window of EM.  8 rows a block of 64 experts 233 -> 294 us, 35
+//   298 -> 330, 44 340 -> 351, 55 397 -> 389, 77 753 -> 584, 96 1310 -> 1089; of 256 experts 26 2045 ->
+//   2153, 43 2557 -> 2438, 64 4157 -> 3803.
+//   Blocks of 16, 32, 64, several experts to a window: 64 rows a segment as well.  Without that an
+//   expert's 12 rows in blocks of 16 were taken (256 experts of 7168 x 2048 2012 -> 2833 us, 64 of 4096
+//   x 1536 436 -> 830); 64 rows in blocks of 16 3142 -> 3292 and 474 -> 484, 96 in blocks of 32 536 ->
+//   563, 64 in blocks of 64 428 -> 441; from the line on 144 in blocks of 16 5154 -> 4866 and 735 -> 670,
+//   in blocks of 32 713 -> 634, 96 in blocks of 64 3106 -> 2711 and 404 -> 391.
+//   Blocks of 48, 80, 96, 112, each a window of its own: 30 rows a block.  36 rows an expert in blocks of
+//   48 2158 -> 2222 and 328 -> 332 us; 48 2870 -> 2833 and 400 -> 396, 64 510 -> 426.
+// And no round of workgroups of twice tile_wide's columns that is nearly empty (8 experts of 4096 x
+// 4096, 4000 rows, second stage 280 workgroups for 256 compute units: 530 -> 548 us).
+constexpr int kMxRawRows = 50, kMxRawSegmentRows = 64, kMxRawBlockRows = 30;
+inline bool mx_raw_pays(long long rows, long long EM, int block_size, int ispp, int hidden) {
+  if (rows * kMxRows < kMxRawRows * EM) return false;
+  const long long padding = EM - rows;
+  long long windows = rows / kMxRows + padding / (2 * (kMxRows - 1)) + 1;
+  if (block_size < kMxRows && padding > 0) {
+    const double run = (double)rows * (block_size - 1) / (double)padding;  // an expert's rows
+    const double padded = run + (block_size - 1) / 2.0;
+    const bool shared = kMxRows % block_size == 0;
+    const double segments = shared ? 1.0 + (padded > block_size ? (padded - block_size) / kMxRows : 0.0)
+                                   : padded / block_size;  // an expert's
+    if (run < segments * (shared ? kMxRawSegmentRows : kMxRawBlockRows)) return false;
+    if (shared) windows = (rows + padding / 2) / kMxRows + 1;
+  }
+  for (int stage = 0; stage < 2; ++stage) {
+    const int units = mx_units(stage, stage == 0 ? ispp : hidden);
+    const long long tiles = windows * ((units + kMxWaves - 1) / kMxWaves);
+    if (5 * tiles < 3 * ((tiles + 255) / 256 * 256)) return false;
+  }
+  return true;
+}
+
 // ---- epilogue staging: a wavefront's own quarter of the ring ----
 __host__ __device__ constexpr inline uint32_t mx_stage_base(int wave, int terms) {
   return (uint32_t)(wave * (kMxRing * mx_slot_bytes(terms) / kMxWaves));
