@@ -157,6 +157,12 @@ void vk_hip_fused_moe_mxfp4_ws(
  * counterpart in the reference.
  */
 #define VK_HIP_MOE_OVERWRITE_OUT 1u
+/* VK_HIP_MOE_MAPPED: sorted_ids / expert_ids were built with an expert map that
+ * leaves experts (and the rows routed to them) to other ranks, so M * top_k says
+ * nothing of how many rows this call multiplies.  A hint on speed: on raw weights
+ * a call then keeps to the kernel that costs least when rows turn out to be few.
+ * (vk_hip_moe_route_layer_mxfp4 sees the map itself.) */
+#define VK_HIP_MOE_MAPPED 16u
 
 void vk_hip_fused_moe_mxfp4_ex(
     const uint16_t* A, const uint8_t* w13, const uint8_t* w13_scale,

@@ -68,11 +68,11 @@ def test_few_rows_a_segment_are_left_to_the_other_kernel(raw_rule, H, I, E, k, b
 
 @pytest.mark.parametrize("block", [16, 48, 64, 128, 256])
 def test_the_rule_takes_any_sizes(raw_rule, block):
-    """... of a valid call: EM below the rows (an expert map drops the others), or far above."""
+    """... of a valid call: EM below the rows (an expert map drops the others; refused), or far above."""
     for rows in (1, 513, 8192, 2 ** 31 - 1):
         for em in (block, rows // 2 // block * block + block, 2 ** 31 - 1):
             for width in (64, 512, 7168):
-                assert raw_rule(rows, em, block, width, width) in (0, 1)
+                assert raw_rule(rows, em, block, width, width) in ((0,) if em < rows else (0, 1))
 
 
 def _weights(E, H, I, gen, special):
@@ -124,3 +124,36 @@ def test_same_bits_as_on_prepacked_weights(H, I, E, k, T, epilogue, special):
     # ... and the raw call is not the slower kernels' (their two FP8 terms round differently)
     again = raw.apply(A, ids, tw, output_dtype=torch.float32)
     assert torch.equal(torch.nan_to_num(a), torch.nan_to_num(again))
+
+
+def _other_kernel(fe):
+    """Has fe's calls run tile_wide_kernel: a workspace too short for the FP4-rate kernels' rows."""
+    size = fe.ws_bytes_fn
+    fe.ws_bytes_fn = lambda *a: size(*a) - 256
+    return fe
+
+
+# A rank's share of the experts: most rows are other ranks', which the rule cannot see in M * top_k
+@pytest.mark.gpu
+@pytest.mark.parametrize("entry", ["apply", "route_layer"])
+def test_mapped_calls_are_left_to_the_other_kernel(entry):
+    H, I, E, k, T, ranks = 1024, 512, 15, 4, 3000, 4
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    w = _weights(E, H, I, gen, False)
+    A = torch.randn((T, H), device="cuda", generator=gen).to(torch.bfloat16)
+    logits = torch.randn((T, E * ranks), device="cuda", generator=gen)
+    local = torch.full((E * ranks,), -1, dtype=torch.int32, device="cuda")
+    local[::ranks] = torch.arange(E, dtype=torch.int32, device="cuda")
+    def call(fe, A, logits):
+        if entry == "route_layer":
+            return fe.route_layer(A, logits, k)[0]
+        ids, tw = fe.route(logits, k)
+        return fe.apply(A, ids, tw, output_dtype=torch.float32)
+    mapped = [call(f(ve.FusedExperts(*w, expert_map=local, local_num_experts=E)), A, logits)
+              for f in (lambda fe: fe, _other_kernel)]
+    assert torch.equal(*mapped)
+    # (without a map the same sizes are the raw form's, which rounds differently)
+    own = logits[:, :E].contiguous()
+    plain = [call(f(ve.FusedExperts(*w)), A, own) for f in (lambda fe: fe, _other_kernel)]
+    assert not torch.equal(*plain)
+    torch.testing.assert_close(*plain, rtol=0, atol=2e-2 * float(plain[1].pow(2).mean().sqrt()))

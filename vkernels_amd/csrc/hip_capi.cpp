@@ -840,6 +840,7 @@ int vk_hip_moe_route_layer_mxfp4(
   a.w13_packed = static_cast<const uint8_t*>(w13_packed);
   a.w2_packed = static_cast<const uint8_t*>(w2_packed);
   a.num_experts = num_local_experts;
+  if (expert_map != nullptr && local_n < num_experts) a.flags |= VK_HIP_MOE_MAPPED;
   if (packed_only && !vk::fused_moe_packed_only_ok(a)) return fail(VK_ERROR_INVALID_ARGUMENT, kPackedOnlyNeeds);
   if (num_experts > 0 && top_k <= num_experts && local_n >= 0 && local_n <= num_experts) {
     vk::RoutedArgs r{};

@@ -1525,7 +1525,12 @@ bool mx_raw_takes(const uint8_t* w, const uint8_t* w_scale, int rows, int K) {
 bool mx_plan(const FusedMoeArgs& a, bool need_stage0, bool raw, MxPlan& pl) {
   if (a.workspace == nullptr) return false;
   if (raw) {
-    if (!mx_raw_pays((long long)a.M * a.top_k, a.EM, a.block_size, a.ispp, a.hidden) || (need_stage0 && !mx_raw_takes(a.w13, a.w13_scale, 2 * a.ispp, a.hidden)) ||
+    // Rows that an expert map leaves to other ranks count in M * top_k (flag 16: VK_HIP_MOE_MAPPED), so
+    // the rule would judge by several times the rows there are.  A rank of four, c4, 1000 tokens: raw
+    // form 180 us, tile_wide_kernel 131; 500 147 and 99; 2000 194 and 243; a rank of eight, c3, 1024
+    // 326 and 300, 4096 663 and 622.
+    if ((a.flags & 16u) != 0u || !mx_raw_pays((long long)a.M * a.top_k, a.EM, a.block_size, a.ispp, a.hidden) ||
+        (need_stage0 && !mx_raw_takes(a.w13, a.w13_scale, 2 * a.ispp, a.hidden)) ||
         !mx_raw_takes(a.w2, a.w2_scale, a.hidden, a.ispp) || a.ispp % 64 != 0)
       return false;
   } else if ((need_stage0 && a.w13_packed == nullptr) || a.w2_packed == nullptr) {

@@ -183,8 +183,8 @@ __host__ __device__ constexpr inline int mx_raw_fix_slot(int live, int terms, in
 // 4096, 4000 rows, second stage 280 workgroups for 256 compute units: 530 -> 548 us).
 constexpr int kMxRawRows = 50, kMxRawSegmentRows = 64, kMxRawBlockRows = 30;
 inline bool mx_raw_pays(long long rows, long long EM, int block_size, int ispp, int hidden) {
-  if (rows * kMxRows < kMxRawRows * EM) return false;
   const long long padding = EM - rows;
+  if (padding < 0 || rows * kMxRows < kMxRawRows * EM) return false;  // (fewer: an expert map drops rows)
   long long windows = rows / kMxRows + padding / (2 * (kMxRows - 1)) + 1;
   if (block_size < kMxRows && padding > 0) {
     const double run = (double)rows * (block_size - 1) / (double)padding;  // an expert's rows

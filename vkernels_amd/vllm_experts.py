@@ -251,6 +251,7 @@ MOE_OVERWRITE_OUT = 1  # VK_HIP_MOE_OVERWRITE_OUT
 MOE_SPLIT2 = 2         # VK_HIP_MOE_SPLIT2
 MOE_W4A4 = 4           # VK_HIP_MOE_W4A4
 MOE_SPLIT3 = 8         # VK_HIP_MOE_SPLIT3
+MOE_MAPPED = 16        # VK_HIP_MOE_MAPPED
 
 
 def resolve_prepack_fns(lib):
@@ -667,6 +668,8 @@ class FusedExperts:
             ws = self.scratch.get(("ws", K, self.ispp), need, dtype=torch.uint8, device=dev,
                                   capacity=cap_bytes, name="workspace")
             flags = MOE_OVERWRITE_OUT if overwrite else 0
+            if self.expert_map is not None and self.local_n < self.global_E:
+                flags |= MOE_MAPPED
             if self.w13_packed is not None:
                 if self.w4a4:
                     flags |= MOE_W4A4
