@@ -26,7 +26,8 @@ def _build(tmp_path, *defines):
 
 def test_offsets_and_schedule(tmp_path):
     exe = _build(tmp_path)
-    for args in ("0 7168 2048 3", "1 2048 7168 3", "0 4096 1536 2", "1 1536 4096 2", "0 512 512 2", "1 512 512 2"):
+    for args in ("0 7168 2048 3", "1 2048 7168 3", "0 4096 1536 2", "1 1536 4096 2", "0 512 512 2", "1 512 512 2",
+                 "1 512 704 2"):  # (the last unit of the last is ragged)
         res = subprocess.run([str(exe), *args.split()], capture_output=True, text=True)
         assert res.returncode == 0, f"{args}: {res.stderr.strip()}"
 
@@ -121,9 +122,9 @@ def test_same_bits_as_on_prepacked_weights(H, I, E, k, T, epilogue, special):
     b = packed.apply(A, ids, tw, output_dtype=torch.float32)
     assert torch.equal(torch.isnan(a), torch.isnan(b))
     assert torch.equal(torch.nan_to_num(a), torch.nan_to_num(b))
-    # ... and the raw call is not the slower kernels' (their two FP8 terms round differently)
-    again = raw.apply(A, ids, tw, output_dtype=torch.float32)
-    assert torch.equal(torch.nan_to_num(a), torch.nan_to_num(again))
+    # ... and it was the raw form that ran: the other kernel's two FP8 terms round differently
+    other = _other_kernel(raw).apply(A, ids, tw, output_dtype=torch.float32)
+    assert not torch.equal(torch.nan_to_num(a), torch.nan_to_num(other))
 
 
 def _other_kernel(fe):
@@ -157,3 +158,60 @@ def test_mapped_calls_are_left_to_the_other_kernel(entry):
     plain = [call(f(ve.FusedExperts(*w)), A, own) for f in (lambda fe: fe, _other_kernel)]
     assert not torch.equal(*plain)
     torch.testing.assert_close(*plain, rtol=0, atol=2e-2 * float(plain[1].pow(2).mean().sqrt()))
+
+
+# Several experts' rows in a window: the ring and each wavefront's scale bytes are used again from one
+# segment to the next; blocks that are windows of their own (48, 112); rows that a map drops
+@pytest.mark.gpu
+@pytest.mark.parametrize("block,dropped", [(16, 0), (32, 0), (48, 0), (64, 0), (112, 0), (256, 0), (16, 7), (64, 7), (128, 7)])
+def test_same_bits_in_other_blocks_and_under_a_map(block, dropped):
+    H, I, E, k, T = 1024, 512, 60, 4, 3000 if block != 256 else 4500
+    gen = torch.Generator(device="cuda").manual_seed(block)
+    w = _weights(E, H, I, gen, True)
+    kw = dict(b13=torch.randn((E, 2 * I), device="cuda", generator=gen), b2=torch.randn((E, H), device="cuda", generator=gen))
+    if dropped:  # experts in another order, a few of them elsewhere
+        perm = torch.randperm(E, device="cuda", generator=gen).to(torch.int32)
+        kw["expert_map"] = torch.where(perm < E - dropped, perm, torch.full_like(perm, -1))
+    A = torch.randn((T, H), device="cuda", generator=gen).to(torch.bfloat16)
+    A[5, 7], A[T - 1, H - 1] = float("inf"), 1e-38
+    logits = torch.randn((T, E), device="cuda", generator=gen)
+    raw, packed = ve.FusedExperts(*w, **kw), ve.FusedExperts(*w, prepack=True, split_terms=3, **kw)
+    ids, tw = raw.route(logits, k)
+    a, b, other = (fe.apply(A, ids, tw, block_size=block, output_dtype=torch.float32).nan_to_num()
+                   for fe in (raw, packed, _other_kernel(ve.FusedExperts(*w, **kw))))
+    assert torch.equal(a, b)
+    assert not torch.equal(a, other)
+
+
+# The second stage alone; a last unit that is ragged (704 = 5 units of 128 and half of one), its bias too
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,block", [(704, 128), (704, 64), (1024, 128)])
+def test_same_bits_of_the_second_stage_alone(H, block):
+    I, E, M = 512, 4, 11000
+    gen = torch.Generator(device="cuda").manual_seed(H)
+    w = _weights(E, H, I, gen, False)
+    b2 = torch.randn((E, H), device="cuda", generator=gen)
+    packed = ve.FusedExperts(*w, prepack=True)
+    ids = torch.randint(0, E, (M, 1), device="cuda", generator=gen).to(torch.int32)
+    tw = torch.rand((M, 1), device="cuda", generator=gen)
+    sids, eids, _, em = packed.align(ids, block)
+    act = torch.randn((em, I), device="cuda", generator=gen).to(torch.bfloat16)
+    need = int(packed.ws_bytes_fn(M, H, I, 1, em))
+    ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+    fn = packed.lib.vk_hip_moe_down_mxfp4_ex
+    fn.restype, P, N = None, ctypes.c_void_p, ctypes.c_int
+    fn.argtypes = [P] * 5 + [N] * 4 + [P, P, N, P, N, P, ctypes.c_size_t, ctypes.c_uint, P, N, P]
+
+    def call(size, w2_packed):
+        out = torch.full((M, H), float("nan"), device="cuda")
+        packed.lib.vk_set_last_error(0, b"")
+        fn(act.data_ptr(), w[2].data_ptr(), w[3].data_ptr(), tw.data_ptr(), out.data_ptr(), M, H, I, 1, sids.data_ptr(),
+           eids.data_ptr(), em, b2.data_ptr(), block, ws.data_ptr(), size, ve.MOE_OVERWRITE_OUT | ve.MOE_SPLIT3,
+           w2_packed, E, torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        assert packed.lib.vk_last_error_code() == 0, ve.last_error(packed.lib)
+        return out
+    raw = call(need, None)
+    assert torch.isfinite(raw).all()
+    assert torch.equal(raw, call(need, packed.w2_packed.data_ptr()))
+    assert not torch.equal(raw, call(need - 256, None))    # (the kernel that takes it in a shorter workspace)

@@ -180,7 +180,8 @@ __host__ __device__ constexpr inline int mx_raw_fix_slot(int live, int terms, in
 //   Blocks of 48, 80, 96, 112, each a window of its own: 30 rows a block.  36 rows an expert in blocks of
 //   48 2158 -> 2222 and 328 -> 332 us; 48 2870 -> 2833 and 400 -> 396, 64 510 -> 426.
 // And no round of workgroups of twice tile_wide's columns that is nearly empty (8 experts of 4096 x
-// 4096, 4000 rows, second stage 280 workgroups for 256 compute units: 530 -> 548 us).
+// 4096, 4000 rows, second stage 280 workgroups for 256 compute units: 530 -> 548 us); a second stage
+// that runs alone is judged as the whole layer is, so it is refused where only the first stage's would be.
 constexpr int kMxRawRows = 50, kMxRawSegmentRows = 64, kMxRawBlockRows = 30;
 inline bool mx_raw_pays(long long rows, long long EM, int block_size, int ispp, int hidden) {
   const long long padding = EM - rows;
