@@ -643,35 +643,24 @@ __device__ __forceinline__ void exact_unit_mx(const MxArgs& p, int e, int unit, 
 // waited for: the caller counts it and passes the registers through wait_loads.
 // A memory operation may read a scalar register that a vector instruction wrote only five
 // wait states later, and the compiler, which keeps that distance otherwise, does not look
-// into inline assembly: where it brings a spilled base back (v_readlane) the operation
-// would take half of an old one.  COPY: the load goes through a copy of its base (a scalar
-// instruction may read the register at once, and the operation the copy).
-template <int OFF, bool COPY>
+// into inline assembly: a spilled base that it brings back (v_readlane) right in front of one
+// would be read half old.  tests/test_inline_loads.py follows every way through the built code
+// for it and finds none: what comes back from a spill goes through a scalar addition first.  A
+// copy of the base in front of each operation, which needs no such check, cost 1000 tokens of c4
+// 299.1 -> 302.0 us a layer and 4096 of c3 on raw weights 3766 -> 3893 (the second stage of the
+// former 79.2 -> 82.3), and 300.7 and 3901 with copies ahead of the K loop only.
+template <int OFF>
 __device__ __forceinline__ void load16_nowait(u32x4& dst, uint32_t voff, const uint8_t* base) {
-  if constexpr (COPY) {
-    uint64_t b;
-    __asm__ volatile("s_mov_b64 %1, %3\n\tglobal_load_dwordx4 %0, %2, %1 offset:%4"
-                     : "=&v"(dst), "=&s"(b) : "v"(voff), "s"(base), "n"(OFF) : "memory");
-  } else {
-    __asm__ volatile("global_load_dwordx4 %0, %1, %2 offset:%3" : "=&v"(dst) : "v"(voff), "s"(base), "n"(OFF) : "memory");
-  }
+  __asm__ volatile("global_load_dwordx4 %0, %1, %2 offset:%3" : "=&v"(dst) : "v"(voff), "s"(base), "n"(OFF) : "memory");
 }
-template <bool COPY>
 __device__ __forceinline__ void load8_nowait(u32x2& dst, uint32_t voff, const uint8_t* base) {
-  if constexpr (COPY) {
-    uint64_t b;
-    __asm__ volatile("s_mov_b64 %1, %3\n\tglobal_load_dwordx2 %0, %2, %1"
-                     : "=&v"(dst), "=&s"(b) : "v"(voff), "s"(base) : "memory");
-  } else {
-    __asm__ volatile("global_load_dwordx2 %0, %1, %2" : "=&v"(dst) : "v"(voff), "s"(base) : "memory");
-  }
+  __asm__ volatile("global_load_dwordx2 %0, %1, %2" : "=&v"(dst) : "v"(voff), "s"(base) : "memory");
 }
 // The DMA form with a uniform base and a 32-bit offset per lane: 16 bytes per lane to
-// LDS at lds_base + 16 * lane.  (The copy of the base is also the wait state behind m0.)
+// LDS at lds_base + 16 * lane.
 __device__ __forceinline__ void dma16_saddr(uint32_t voff, const uint8_t* base, uint32_t lds_base) {
-  uint64_t b;
-  __asm__ volatile("s_mov_b32 m0, %1\n\ts_mov_b64 %0, %3\n\tglobal_load_lds_dwordx4 %2, %0"
-                   : "=&s"(b)
+  __asm__ volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                   :
                    : "s"(__builtin_amdgcn_readfirstlane(lds_base)), "v"(voff), "s"(base)
                    : "memory");
 }
@@ -679,10 +668,10 @@ __device__ __forceinline__ void dma16_saddr(uint32_t voff, const uint8_t* base, 
 // The same in all lanes (mask ~0) or in none (0; uniform), without a branch: one in the K loop makes
 // the register allocator shuffle accumulators.
 __device__ __forceinline__ void dma16_masked(uint32_t mask, uint32_t voff, const uint8_t* base, uint32_t lds_base) {
-  uint64_t exec, b;
-  __asm__ volatile("s_mov_b64 %0, exec\n\ts_mov_b32 exec_lo, %5\n\ts_mov_b32 exec_hi, %5\n\ts_mov_b32 m0, %2\n\t"
-                   "s_mov_b64 %1, %4\n\tglobal_load_lds_dwordx4 %3, %1\n\ts_mov_b64 exec, %0"
-                   : "=&s"(exec), "=&s"(b)
+  uint64_t exec;
+  __asm__ volatile("s_mov_b64 %0, exec\n\ts_mov_b32 exec_lo, %4\n\ts_mov_b32 exec_hi, %4\n\ts_mov_b32 m0, %1\n\t"
+                   "s_nop 0\n\tglobal_load_lds_dwordx4 %2, %3\n\ts_mov_b64 exec, %0"
+                   : "=&s"(exec)
                    : "s"(__builtin_amdgcn_readfirstlane(lds_base)), "v"(voff), "s"(base),
                      "s"(__builtin_amdgcn_readfirstlane(mask))
                    : "memory");
@@ -860,39 +849,31 @@ __global__ __launch_bounds__(64 * kMxWaves) void tile_mx_kernel(MxArgs p) {
       dma16_saddr(cp_off[g] + mx_row_copy_step_offset(term, Kp, step, nsteps), p.Aq,
                   lds_base + mx_row_copy_lds(step, wave, TERMS, term, g));
     };
-    // ---- weight loads.  Ahead of the K loop the compiler brings some bases back from a spill, so they
-    // are copied; inside it scalar instructions make each step's base anew (tests/test_inline_loads.py
-    // follows every way through the built code for it).  Copies there as well, 27 of 781 instructions
-    // of three steps, cost 1000 tokens of c4 300.4 -> 302.5 us a layer, 500 of c4 221.2 -> 223.1, 2048
-    // of c1 405.7 -> 407.3, 4096 of c2 858.9 -> 861.5; the even spread of the loads over the first
-    // stage's steps, timed apart from them, is within 0.5 % of two or three loads at a time.
-    constexpr IntC<1> kAhead{};
-    constexpr IntC<0> kInLoop{};
+    // ---- weight loads
     const uint8_t* wp_unit = p.Wp + mx_unit_offset(e, p.units, unit, nsteps);
     const uint32_t voff16 = (uint32_t)lane * 16u, voff8 = (uint32_t)lane * 8u;
-    auto load_weights = [&](auto copy_c, WeightStep& ws, int step, int j) {  // operation j (0 .. 8)
-      constexpr bool COPY = decltype(copy_c)::value != 0;
+    auto load_weights = [&](WeightStep& ws, int step, int j) {  // operation j (0 .. 8)
       const uint8_t* base = wp_unit + mx_step_offset(step, nsteps);
       // (the immediates and lane offsets below are mx_weight_load_offset(j, lane))
       static_assert(mx_weight_load_offset(3, 2) == 3072 + 32 && mx_weight_load_offset(6, 0) == 4096 + 2048 &&
                         mx_weight_load_offset(8, 3) == 8192 + 24,
                     "weight loads and their layout function disagree");
       switch (j) {
-        case 0: load16_nowait<0, COPY>(ws.w[0], voff16, base); break;
-        case 1: load16_nowait<1024, COPY>(ws.w[1], voff16, base); break;
-        case 2: load16_nowait<2048, COPY>(ws.w[2], voff16, base); break;
-        case 3: load16_nowait<3072, COPY>(ws.w[3], voff16, base); break;
-        case 4: load16_nowait<0, COPY>(ws.w[4], voff16, base + 4096); break;
-        case 5: load16_nowait<1024, COPY>(ws.w[5], voff16, base + 4096); break;
-        case 6: load16_nowait<2048, COPY>(ws.w[6], voff16, base + 4096); break;
-        case 7: load16_nowait<3072, COPY>(ws.w[7], voff16, base + 4096); break;
-        default: load8_nowait<COPY>(ws.sc, voff8, base + 8192); break;
+        case 0: load16_nowait<0>(ws.w[0], voff16, base); break;
+        case 1: load16_nowait<1024>(ws.w[1], voff16, base); break;
+        case 2: load16_nowait<2048>(ws.w[2], voff16, base); break;
+        case 3: load16_nowait<3072>(ws.w[3], voff16, base); break;
+        case 4: load16_nowait<0>(ws.w[4], voff16, base + 4096); break;
+        case 5: load16_nowait<1024>(ws.w[5], voff16, base + 4096); break;
+        case 6: load16_nowait<2048>(ws.w[6], voff16, base + 4096); break;
+        case 7: load16_nowait<3072>(ws.w[7], voff16, base + 4096); break;
+        default: load8_nowait(ws.sc, voff8, base + 8192); break;
       }
     };
     // operation k (0 .. kOps - 1) of what a K step issues for step `step`
-    auto issue = [&](auto copy_c, WeightStep& ws, int step, int k) {
+    auto issue = [&](WeightStep& ws, int step, int k) {
       if (k < kRowOps) copy_rows(step, k);
-      else load_weights(copy_c, ws, step, k - kRowOps);
+      else load_weights(ws, step, k - kRowOps);
     };
 
     // ---- operand reads: lane (ln, hh) takes block 2 half + hh of row ln of row tile m:
@@ -951,9 +932,9 @@ __global__ __launch_bounds__(64 * kMxWaves) void tile_mx_kernel(MxArgs p) {
       // prologue: the loads of steps 0 and 1; step 0's have landed in every wavefront
       // once only step 1's are outstanding
 #pragma unroll
-      for (int k = 0; k < kOps; ++k) issue(kAhead, ws[0], 0, k);
+      for (int k = 0; k < kOps; ++k) issue(ws[0], 0, k);
 #pragma unroll
-      for (int k = 0; k < kOps; ++k) issue(kAhead, ws[1], 1, k);
+      for (int k = 0; k < kOps; ++k) issue(ws[1], 1, k);
       wait_loads<kOps>(ws[0]);
       __builtin_amdgcn_s_barrier();
       __asm__ volatile("" ::: "memory");
@@ -976,7 +957,7 @@ __global__ __launch_bounds__(64 * kMxWaves) void tile_mx_kernel(MxArgs p) {
           auto issue_at = [&](int t) {
 #pragma unroll
             for (int k = 0; k < kOps; ++k)
-              if (mx_op_slot(LIVE, TERMS, k) == 4 * q + t) issue(kInLoop, ws[in2], c + 2, k);
+              if (mx_op_slot(LIVE, TERMS, k) == 4 * q + t) issue(ws[in2], c + 2, k);
           };
           // (a wavefront without a unit multiplies unit 0's weights and drops the result)
           acc[m][0] = mfma_fp4_act<0, TERMS == 1, kRowsFirst>(ws[i].w[half * 4 + 0], cur, acc[m][0], wsc);
@@ -1081,8 +1062,8 @@ __global__ __launch_bounds__(64 * kMxWaves) void tile_mx_kernel(MxArgs p) {
         dst = fp4x8_to_ocp_doubled(w);
       };
       // operation k (0 .. kHalfOps - 1) of a half step, for half step `half` of K step `step`
-      auto issue_raw = [&](auto copy_c, WeightHalf& h, int step, int half, int k) {
-        if (k < 4) load16_nowait<0, decltype(copy_c)::value != 0>(h.w[k], w_off[k], w_base + mx_raw_load_offset(step, nsteps, half));
+      auto issue_raw = [&](WeightHalf& h, int step, int half, int k) {
+        if (k < 4) load16_nowait<0>(h.w[k], w_off[k], w_base + mx_raw_load_offset(step, nsteps, half));
         else copy_rows(step, half * (kHalfOps - 4) + k - 4);
       };
       auto base_of = [&](int slot_) {
@@ -1103,7 +1084,7 @@ __global__ __launch_bounds__(64 * kMxWaves) void tile_mx_kernel(MxArgs p) {
       copy_scales(0, ~0u);
       static_for<4>([&](auto s_c) {
 #pragma unroll
-        for (int k = 0; k < kHalfOps; ++k) issue_raw(kAhead, hs[decltype(s_c)::value], decltype(s_c)::value >> 1, decltype(s_c)::value & 1, k);
+        for (int k = 0; k < kHalfOps; ++k) issue_raw(hs[decltype(s_c)::value], decltype(s_c)::value >> 1, decltype(s_c)::value & 1, k);
       });
       wait_half<2 * kHalfOps>(hs[0]);
       wait_half<2 * kHalfOps>(hs[1]);
@@ -1137,7 +1118,7 @@ __global__ __launch_bounds__(64 * kMxWaves) void tile_mx_kernel(MxArgs p) {
             if constexpr (t == 2) __asm__ volatile("" : "+v"(nxt));  // complete from here on (read a group ago)
             static_for<kHalfOps>([&](auto k_c) {
               if constexpr (mx_raw_op_slot(LIVE, TERMS, decltype(k_c)::value) == 4 * (q - half * G) + t)
-                issue_raw(kInLoop, hs[mx_raw_weight_set(2 * i + half)], c + 2, half, decltype(k_c)::value);
+                issue_raw(hs[mx_raw_weight_set(2 * i + half)], c + 2, half, decltype(k_c)::value);
             });
             static_for<16>([&](auto x_c) {
               constexpr int x = decltype(x_c)::value;
