@@ -123,10 +123,18 @@ void vk_hip_fused_moe_mxfp4(
  * callers that can provide one (the library itself allocates nothing).  With
  * at least vk_hip_fused_moe_mxfp4_workspace_bytes(M, hidden, ispp, top_k, EM)
  * bytes, 16-byte aligned, the prefill-sized path splits the bf16 rows into their
- * FP8 terms once per call instead of once per workgroup, and its second stage
+ * terms once per call instead of once per workgroup, and its second stage
  * stores its rows (fp32, [EM, hidden], the bulk of the workspace) for a last pass
  * that sums each token's rows in selection order, instead of one atomic add per
- * row and column; results agree to fp32 rounding.
+ * row and column; results agree to fp32 rounding where the terms are the same.
+ * The terms are two FP8 ones or, where the matrix cores' FP4 rate pays, three FP6 ones as in the prepacked call with
+ * VK_HIP_MOE_SPLIT3 (the same bits): weights and scales 16-byte aligned, hidden and
+ * ispp multiples of 512, and rows enough for the blocks they are in (about 80 an
+ * expert in blocks of 128, 120 in blocks of 16).  Against the layer in 64-bit sums
+ * the second is no further off (8e-5 and 1.4e-4 relative L2), but a caller that
+ * compares calls of different M bit by bit sees the change.  The flags that choose
+ * terms (VK_HIP_MOE_SPLIT2, VK_HIP_MOE_SPLIT3, VK_HIP_MOE_W4A4) are about
+ * prepacked weights and change nothing on raw ones.
  * A null or short workspace is vk_hip_fused_moe_mxfp4 exactly.  The contents
  * of the workspace are unspecified after the call; calls that share one
  * must be ordered on a stream.  No counterpart in the reference, whose Python

@@ -34,8 +34,9 @@
 //   scale bytes then come with the codes and nothing is checked or moved in the
 //   loop), and forms that align, or route and align, for themselves.
 // tile_wide_kernel: everything else when the caller lends a workspace (and K >=
-//   512) that moe_prefill.hip does not take on the raw tensors: 128 rows x 16 weight tiles per workgroup, rows pre-split in the
-//   workspace, operands brought to LDS by DMA three K steps ahead; the second
+//   512) that moe_prefill.hip does not take on the raw tensors (mx_raw_pays in
+//   moe_prefill_layout.hpp): 128 rows x 16 weight tiles per workgroup, rows pre-split
+//   in the workspace, operands brought to LDS by DMA three K steps ahead; the second
 //   stage stores its rows and combine_kernel sums them per token.
 // tile_gemm_kernel: everything else without a workspace: 64 rows x 16 weight
 //   tiles per workgroup, K in chunks of 512, rows split in-kernel.

@@ -736,9 +736,6 @@ __device__ __forceinline__ f32x16 mfma_fp4_act(u32x4 w, i32x8 b, f32x16 acc, uin
                                                            (int)wscale, 0, b[W4A4 ? 4 : 6]);
 }
 
-// PREACT: the stage's linear part alone (tensor-parallel callers sum it over their K slices
-// before the epilogue): the accumulators of the routed rows go to p.preact as fp32, no
-// bias, no activation, no routing weight; rows that are not routed are left as they are.
 // f(IntC<0>), ..., f(IntC<N - 1>): indices that are constants before anything is unrolled.
 template <int N, int I = 0, typename F>
 __device__ __forceinline__ void static_for(F f) {
@@ -748,6 +745,9 @@ __device__ __forceinline__ void static_for(F f) {
   }
 }
 
+// PREACT: the stage's linear part alone (tensor-parallel callers sum it over their K slices
+// before the epilogue): the accumulators of the routed rows go to p.preact as fp32, no
+// bias, no activation, no routing weight; rows that are not routed are left as they are.
 // RAW: the weights as the checkpoint has them (p.W, p.Ws), moved onto the code points and checked
 // in the loop.
 template <int STAGE, int TERMS, bool PREACT = false, bool RAW = false>
@@ -1005,13 +1005,18 @@ __global__ __launch_bounds__(64 * kMxWaves) void tile_mx_kernel(MxArgs p) {
       wait_loads<0>(ws[2]);
     };
     // The same on raw weights.  A lane's 16 bytes lie in a line of their own, so an operand load
-    // occupies the memory pipe 75 cycles instead of 18 (measured, 4 wavefronts): 8 of them, the
-    // row copies and the scale bytes are 3.3 k cycles a step of 3.1 k cycles of MFMAs, whatever
-    // the live rows.  4096 tokens of 256 experts of 7168 x 2048: 2622 -> 2190 us this stage and
-    // 1412 -> 1280 us the second against tile_wide_kernel; 64 experts of 4096 x 1536: 774 -> 585
-    // and 452 -> 350 us.  (Loads of 16 rows x 64 bytes, 37 cycles each, put in order by a lane
-    // permutation through LDS and row swaps, were 1 to 4 % behind at these sizes and ahead where
-    // this form is not taken.)
+    // occupies the memory pipe 75 cycles instead of 18 (measured alone, 4 wavefronts): with the row
+    // copies and the scale bytes 3.3 k cycles a step, whatever the live rows, beside 3.1 k cycles of
+    // MFMAs at four row tiles.  A step takes more than either, some 6 k cycles (4096 tokens of 256
+    // experts of 7168 x 2048: 4.35 M cycles at 1.92 GHz for 12 rounds of 56 steps, half of them
+    // with few rows).  Not separated by measurement: every line is asked for in four half steps and
+    // the 64 KiB of lines of four wavefronts exceed the vector cache; the form needs more registers
+    // than there are (19 and 38 spilled, none that a load in flight writes), and for one of them
+    // the compiler waits for all loads in the second stage's loop of three row tiles.
+    // Against tile_wide_kernel: these sizes 2551 -> 2240 us this stage and 1373 -> 1300 us the
+    // second; 64 experts of 4096 x 1536: 729 -> 597 and 440 -> 342 us.  (Loads of 16 rows x 64 bytes,
+    // 37 cycles each, put in order by a lane permutation through LDS and row swaps, were 1 to 4 %
+    // behind at these sizes and ahead where this form is not taken.)
     auto raw_loop = [&](auto live_c) {
       constexpr int LIVE = decltype(live_c)::value;
       constexpr int G = mx_raw_groups(LIVE, TERMS), Q = 2 * G, kHalfOps = mx_raw_ops(TERMS);
@@ -1182,8 +1187,10 @@ __global__ __launch_bounds__(64 * kMxWaves) void tile_mx_kernel(MxArgs p) {
     // ---- epilogue.  fp32 rows (kRowsFirst): lane (ln, hh) holds, of column ln of each tile, rows
     // 8 (i / 4) + 4 hh + i % 4 of the row tile; a store instruction writes two whole lines of 32
     // columns, straight from the accumulators.  Without the way through LDS, and with the loop's
-    // loads spread evenly, the second stage of 16384 x 8 rows of 2048 x 7168 takes 2.39 instead of
-    // 2.50 ms, of 4096 x 4 of 2880 x 2880 245 instead of 260 us; of 1000 x 6 of 1536 x 4096 level.
+    // loads spread evenly, the second stage of 16384 x 8 rows of 2048 x 7168 takes 2.32 instead of
+    // 2.47 ms, of 4096 x 4 of 2880 x 2880 227 instead of 241 us, of 1000 x 6 of 1536 x 4096 85 instead
+    // of 87.  (With the stores as they are and the loads two or three at a time 2.45 ms and 227 us
+    // against 2.35 and 222 spread, in a run of their own.)
     // Activations (the same there is 1 to 3 % longer: arithmetic takes the time, not the stores):
     // lane (ln, hh) holds, of row 32 m + ln, columns 8 (i / 4) + 4 hh + i % 4 of each tile; the
     // values of 32 rows go through a staging area of the wavefront's own in the ring (free after
